@@ -4,11 +4,11 @@
 //   wrap + ghost images (count, scan, fill)          neighbor.hip
 //   cell binning (count, scan, scatter)              neighbor.hip
 //   sel-sorted neighbour list                        neighbor.hip
-//   env mat + embedding + contraction -> Tsec        embed.hip   (FP64 MFMA)
-//   descriptor T, D                                  embed.hip
+//   env mat + embedding + contraction -> T           expand.hip  (FP64 MFMA;
+//     nets without a short expansion: embed.hip, and the sections' sum there)
 //   fitting forward + input gradient per type        fitting.hip (FP64 MFMA)
 //   dE/dD -> dE/dT                                   fitting.hip
-//   embedding backward -> edge gradients             embed.hip   (FP64 MFMA)
+//   embedding backward -> edge gradients             expand.hip or embed.hip
 //   reverse list + force / atom-virial gather        force.hip
 //   energy / virial reduction                        force.hip
 // The LAMMPS path replaces the first three stages with sel formatting of the
@@ -32,6 +32,7 @@
 #include <vector>
 
 #include "../../include/dp_amd.h"
+#include "expand.h"
 #include "fixed.h"
 #include "kernels.h"
 #include "model.h"
@@ -82,6 +83,16 @@ struct dp_model {
   double* d_envp = nullptr;
   double* d_tpad = nullptr;
   void* d_fit = nullptr;
+  // the embedding nets' expansion (expand.h): H groups of 64 terms (0: some
+  // net has none, the nets are evaluated slot by slot), the coefficients in
+  // both operand orders, a padded slot's basis values, and the nets as in the
+  // model file (fp64, for slots outside its range)
+  int exp_h = 0;
+  std::vector<int> exp_blocks;
+  double* d_exp_f = nullptr;
+  double* d_exp_b = nullptr;
+  double* d_exp_pad = nullptr;
+  double* d_nets = nullptr;
   // fp64: the first fitting layer's weights of every type transposed,
   // [nt][F0][L3 axis] (the fused dE/dD -> dE/dT kernel's operand), or null
   double* d_w0t = nullptr;
@@ -344,7 +355,7 @@ DescArgs desc_args(dp_model* M, void* Tt, void* D) {
   da.tpad = M->d_tpad;
   da.Tt = Tt;
   da.D = D;
-  da.from_tt = m.ntypes == 1;  // the forward wrote T itself
+  da.from_tt = m.ntypes == 1 || M->exp_h > 0;  // the forward wrote T itself
   return da;
 }
 
@@ -354,6 +365,53 @@ void reduce_outputs(dp_model* M, hipStream_t st, int nloc, int ntarget, const do
                     int ne, const int* items, const Outputs& out);
 void atom_energy_out(dp_model* M, hipStream_t st, int ntarget, const double* e_vals, int ne,
                      const int* items, const Outputs& out);
+
+// The expanded nets' kernel arguments, from the slot-by-slot kernels' bundle.
+void expand_args(const dp_model* M, const EmbArgs& ea, ExpandArgs& xa) {
+  const ModelHost& m = M->host;
+  const int nt = m.ntypes;
+  xa.ntypes = nt;
+  xa.nnei = ea.nnei;
+  int waves = 0;
+  for (int t = 0; t < nt; ++t) {
+    xa.sel[t] = ea.sel[t];
+    xa.wave_off[t] = waves;
+    waves += (ea.type_off[t + 1] - ea.type_off[t] + 3) / 4;
+  }
+  xa.wave_off[nt] = waves;
+  for (int t = 0; t <= nt; ++t) {
+    xa.sec[t] = ea.sec[t];
+    xa.type_off[t] = ea.type_off[t];
+  }
+  for (int k = 0; k < 3; ++k) xa.emb[k] = m.emb[k];
+  for (int p = 0; p < nt * nt; ++p) xa.blocks[p] = (unsigned char)M->exp_blocks[p];
+  xa.rcut = ea.rcut;
+  xa.rcut_smth = ea.rcut_smth;
+  xa.inv_sw = ea.inv_sw;
+  xa.inv_nnei = ea.inv_nnei;
+  xa.fix_gmax = ea.fix_gmax;
+  xa.envp = ea.envp;
+  xa.cf = M->d_exp_f;
+  xa.cb = M->d_exp_b;
+  xa.cf_stride = expand_fwd_stride(M->exp_h, m.emb[2]);
+  xa.cb_stride = expand_bwd_stride(M->exp_h, m.emb[2]);
+  xa.phi_pad = M->d_exp_pad;
+  xa.nets = M->d_nets;
+  xa.net_stride = m.emb_block;
+  xa.ext = ea.ext;
+  xa.nlist = ea.nlist;
+  xa.nreal = ea.nreal;
+  xa.items = ea.items;
+  xa.ldt = ea.ldt;
+  xa.dT = ea.dT;
+  xa.edge_grad = ea.edge_grad;
+  xa.facc = ea.facc;
+  xa.vacc = ea.vacc;
+  xa.cpart = ea.cpsec;
+  xa.zero_n = ea.zero_n;
+  xa.zero_count = ea.zero_count;
+  xa.status = ea.status;
+}
 
 // nall: extended atoms, or (d_nall non-null, standalone path) their
 // capacity with the count itself on the device.
@@ -369,7 +427,8 @@ void run_model_t(dp_model* M, hipStream_t st, int nloc, int nall, const int* d_n
   const int* nreal = static_cast<const int*>(M->nreal.p);
   const int* items = static_cast<const int*>(M->items.p);
 
-  E* Tsec = need<E>(M, M->Tsec, (size_t)nloc * nt * 4 * L3);
+  const bool expand = M->exp_h > 0;
+  E* Tsec = expand ? nullptr : need<E>(M, M->Tsec, (size_t)nloc * nt * 4 * L3);
   // T column-major in bucket order; with axis 16 the first fitting GEMM forms
   // D from it, otherwise D is stored
   E* Tt = need<E>(M, M->Tt, (size_t)std::max(nb, 1) * 4 * L3);
@@ -404,11 +463,17 @@ void run_model_t(dp_model* M, hipStream_t st, int nloc, int nall, const int* d_n
                           ? need<double>(M, M->edge_grad, (size_t)std::max(nloc, 1) * nnei * 3)
                           : nullptr;
   const long nfix = std::max(nall, ntarget);
-  auto* facc = need<unsigned long long>(M, M->facc, (size_t)std::max(nfix, 1L) * 3);
-  auto* vacc = out.atom_virial
-                   ? need<unsigned long long>(M, M->vacc, (size_t)std::max(nfix, 1L) * 9)
-                   : nullptr;
-  double* cpsec = need<double>(M, M->cpsec, (size_t)std::max(nloc, 1) * nt * 12);
+  // words per atom of the fixed-point sums: the expanded nets' backward issues
+  // the values of an edge together, in one array of aligned rows
+  const int fs = !expand ? 3 : out.atom_virial ? 16 : 4, vs = expand ? 16 : 9;
+  auto* facc = need<unsigned long long>(M, M->facc, (size_t)std::max(nfix, 1L) * fs);
+  auto* vacc = !out.atom_virial ? nullptr
+               : expand ? facc + 4
+                        : need<unsigned long long>(M, M->vacc, (size_t)std::max(nfix, 1L) * 9);
+  // own sums per (centre, section); the expanded nets' backward keeps them
+  // per centre
+  const int nsec = expand ? 1 : nt;
+  double* cpsec = need<double>(M, M->cpsec, (size_t)std::max(nloc, 1) * nsec * 12);
 
   EmbArgs ea{};
   ea.ntypes = nt;
@@ -437,6 +502,8 @@ void run_model_t(dp_model* M, hipStream_t st, int nloc, int nall, const int* d_n
   ea.edge_grad = edge_grad;
   ea.facc = facc;
   ea.vacc = vacc;
+  ea.fs = fs;
+  ea.vs = vs;
   ea.cpsec = cpsec;
   // the fixed-point sums are cleared by the forward (no kernel of their own;
   // stores, not a memset, so the step can be captured in a graph); on the
@@ -457,7 +524,11 @@ void run_model_t(dp_model* M, hipStream_t st, int nloc, int nall, const int* d_n
     // fp64: the forward saves the layer-2/3 activations for the backward;
     // mixed precision recomputes them there (no buffer)
     const size_t blk = 16 * (size_t)(M->el.L2P + M->el.L3P);
-    ea.act = f32 ? nullptr : need<E>(M, M->act, (size_t)std::max(nloc, 1) * acc * blk);
+    // (the no-allocation entry point carves it in either case, so that the
+    // systems it accepts do not depend on the model's weights)
+    ea.act = f32 || (expand && !M->arena_on)
+                 ? nullptr
+                 : need<E>(M, M->act, (size_t)std::max(nloc, 1) * acc * blk);
   }
   // Blocks of WAVES * ipw items: each block stages its pair's net in LDS once
   // and its waves then walk ipw items each, which amortises the staging and
@@ -486,16 +557,23 @@ void run_model_t(dp_model* M, hipStream_t st, int nloc, int nall, const int* d_n
     return acc;
   };
 
-  int nblk = block_table(embed_waves_fwd(M->el, f32));
-  launch_embed_fwd(st, M->el, ea, nblk, f32);
+  ExpandArgs xa{};
+  if (expand) expand_args(M, ea, xa);
+  int nblk = expand ? xa.wave_off[nt] : block_table(embed_waves_fwd(M->el, f32));
+  if (expand) {
+    xa.Tt = Tt;
+    launch_expand_fwd(st, xa, M->exp_h, f32);
+  } else {
+    launch_embed_fwd(st, M->el, ea, nblk, f32);
+  }
   if (nblk <= 0) {
     // no forward grid to clear the fixed-point sums (no centres)
-    launch_zero_u64(st, ea.zero_n, ea.zero_count, 3, facc);
-    if (vacc) launch_zero_u64(st, ea.zero_n, ea.zero_count, 9, vacc);
+    launch_zero_u64(st, ea.zero_n, ea.zero_count, fs, facc);
+    if (vacc && !expand) launch_zero_u64(st, ea.zero_n, ea.zero_count, vs, vacc);
   }
   record(M, st, kStEmbFwd + 1);
 
-  if (nt > 1 || D) launch_descriptor(st, desc_args(M, Tt, D), f32);
+  if ((nt > 1 && !expand) || D) launch_descriptor(st, desc_args(M, Tt, D), f32);
   record(M, st, kStDescr + 1);
 
   int active = 0;
@@ -606,23 +684,28 @@ void run_model_t(dp_model* M, hipStream_t st, int nloc, int nall, const int* d_n
   record(M, st, kStDT + 1);
 
   // (the fixed-point sums were cleared by the forward)
-  nblk = block_table(embed_waves_bwd(M->el, f32));
-  launch_embed_bwd(st, M->el, ea, nblk, f32);
+  if (expand) {
+    launch_expand_bwd(st, xa, M->exp_h, f32);
+  } else {
+    nblk = block_table(embed_waves_bwd(M->el, f32));
+    launch_embed_bwd(st, M->el, ea, nblk, f32);
+  }
   M->eg_valid = edge_grad != nullptr;
   record(M, st, kStEmbBwd + 1);
-  const int nsec = nt;
   const unsigned long long *fsum = facc, *vsum = vacc;
   if (d_mapping && ntarget == nloc) {
     // every owner is local: ghost sums folded in place
-    launch_fold_fixed(st, nloc, nall, d_nall, d_mapping, facc, vacc, facc, vacc);
+    launch_fold_fixed(st, nloc, nall, d_nall, d_mapping, fs, vs, facc, vacc, facc, vacc);
   } else if (d_mapping) {
     // owners beyond the locals (the edge graph's kept ghost nodes) share
     // indices with extended atoms: fold every atom into separate target sums
-    auto* ft = need<unsigned long long>(M, M->ftgt, (size_t)std::max(ntarget, 1) * 3);
-    auto* vt = vacc ? need<unsigned long long>(M, M->vtgt, (size_t)std::max(ntarget, 1) * 9) : nullptr;
-    launch_zero_u64(st, ntarget, nullptr, 3, ft);
-    if (vt) launch_zero_u64(st, ntarget, nullptr, 9, vt);
-    launch_fold_fixed(st, 0, nall, d_nall, d_mapping, facc, vacc, ft, vt);
+    auto* ft = need<unsigned long long>(M, M->ftgt, (size_t)std::max(ntarget, 1) * fs);
+    auto* vt = !vacc ? nullptr
+               : expand ? ft + 4
+                        : need<unsigned long long>(M, M->vtgt, (size_t)std::max(ntarget, 1) * vs);
+    launch_zero_u64(st, ntarget, nullptr, fs, ft);
+    if (vt && !expand) launch_zero_u64(st, ntarget, nullptr, vs, vt);
+    launch_fold_fixed(st, 0, nall, d_nall, d_mapping, fs, vs, facc, vacc, ft, vt);
     fsum = ft;
     vsum = vt;
   }
@@ -632,7 +715,7 @@ void run_model_t(dp_model* M, hipStream_t st, int nloc, int nall, const int* d_n
       need<double>(M, M->partials, (size_t)finalize_ev_blocks(ntarget, nloc, nb) * 10);
   double* out10 = need<double>(M, M->out10, 10);
   launch_finalize_ev(st, ntarget, nloc, nb, nsec, static_cast<const int*>(M->ext_type.p), cpsec,
-                     fsum, vsum, e_bucket, out.force, out.atom_virial, partials, out10, out.energy,
+                     fs, vs, fsum, vsum, e_bucket, out.force, out.atom_virial, partials, out10, out.energy,
                      out.virial);
   record(M, st, kStForce + 1);
   atom_energy_out(M, st, ntarget, e_bucket, nb, items, out);
@@ -1293,6 +1376,15 @@ int dp_create(const char* path, int gpu_rank, const void* file_content, size_t c
     };
     upload(M->d_envp, envp);
     upload(M->d_tpad, tpad);
+    ExpandHost ex;
+    if (build_expansion(m, ex)) {
+      M->exp_h = ex.H;
+      M->exp_blocks = ex.blocks;
+      upload(M->d_exp_f, ex.fwd);
+      upload(M->d_exp_b, ex.bwd);
+      upload(M->d_exp_pad, ex.phi_pad);
+      upload(M->d_nets, m.emb_params);
+    }
     if (mixed) {
       // the nets are evaluated in fp32: round the parameters once here
       std::vector<float> emb32(emb.begin(), emb.end());
@@ -1354,7 +1446,9 @@ void dp_destroy(dp_model* M) {
   for (Buf* b : M->bufs)
     if (b->p) (void)hipFree(b->p);
   for (void* p : {M->d_emb, static_cast<void*>(M->d_envp), static_cast<void*>(M->d_tpad), M->d_fit,
-                  M->d_fitf, M->d_c4, static_cast<void*>(M->d_w0t)})
+                  M->d_fitf, M->d_c4, static_cast<void*>(M->d_w0t), static_cast<void*>(M->d_exp_f),
+                  static_cast<void*>(M->d_exp_b), static_cast<void*>(M->d_exp_pad),
+                  static_cast<void*>(M->d_nets)})
     if (p) (void)hipFree(p);
   if (M->async_pending) (void)hipStreamSynchronize(M->async_stream);
   for (auto& set : M->ev)

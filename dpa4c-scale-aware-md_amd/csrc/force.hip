@@ -30,7 +30,8 @@ namespace dpamd {
 // order.
 __global__ __launch_bounds__(256) void k_finalize_ev(int ntarget, int nloc, int nbucket, int nsec,
                                                      const int* __restrict__ type,
-                                                     const double* __restrict__ cpsec,
+                                                     const double* __restrict__ cpsec, int fs,
+                                                     int vs,
                                                      const unsigned long long* __restrict__ facc,
                                                      const unsigned long long* __restrict__ vacc,
                                                      const double* __restrict__ e_bucket,
@@ -52,10 +53,10 @@ __global__ __launch_bounds__(256) void k_finalize_ev(int ntarget, int nloc, int 
   }
   if (t < ntarget) {
 #pragma unroll
-    for (int c = 0; c < 3; ++c) force[3L * t + c] = own[c] - from_fixed(facc[3L * t + c]);
+    for (int c = 0; c < 3; ++c) force[3L * t + c] = own[c] - from_fixed(facc[(long)fs * t + c]);
     if (atom_virial) {
 #pragma unroll
-      for (int q = 0; q < 9; ++q) atom_virial[9L * t + q] = from_fixed(vacc[9L * t + q]);
+      for (int q = 0; q < 9; ++q) atom_virial[9L * t + q] = from_fixed(vacc[(long)vs * t + q]);
     }
   }
   double part[10];
@@ -82,23 +83,25 @@ __global__ __launch_bounds__(256) void k_finalize_ev(int ntarget, int nloc, int 
 }
 
 // Sums of extended atoms j in [j0, n) added onto their owners mapping[j] in
-// dst (which may be src itself when every owner is below j0).
+// dst (which may be src itself when every owner is below j0). Consecutive
+// threads take the values of one atom (P of them a row: three force values,
+// with virials nine more from 4 on), so their atomics share a request (the
+// memory system takes about 24 G atomic requests a second on gfx950 however
+// many lanes a request carries).
+template <int P>
 __global__ __launch_bounds__(256) void k_fold_fixed(int j0, int cap, const int* __restrict__ d_count,
-                                                    const int* __restrict__ mapping,
+                                                    const int* __restrict__ mapping, int fs, int vs,
                                                     const unsigned long long* src_f,
                                                     const unsigned long long* src_v,
                                                     unsigned long long* dst_f,
                                                     unsigned long long* dst_v) {
   const int n = d_count ? *d_count : cap;
-  const int j = j0 + blockIdx.x * blockDim.x + threadIdx.x;
+  const int q = threadIdx.x % P;
+  const long j = j0 + (long)blockIdx.x * (256 / P) + threadIdx.x / P;
   if (j >= n) return;
   const long t = mapping[j];
-#pragma unroll
-  for (int c = 0; c < 3; ++c) atomicAdd(dst_f + 3 * t + c, src_f[3L * j + c]);
-  if (src_v) {
-#pragma unroll
-    for (int q = 0; q < 9; ++q) atomicAdd(dst_v + 9 * t + q, src_v[9L * j + q]);
-  }
+  if (q < 3) atomicAdd(dst_f + fs * t + q, src_f[fs * j + q]);
+  if (P > 4 && q >= 4 && q < 13) atomicAdd(dst_v + vs * t + q - 4, src_v[vs * j + q - 4]);
 }
 
 __global__ __launch_bounds__(256) void k_zero_u64(long cap, const int* __restrict__ d_count,
@@ -109,11 +112,14 @@ __global__ __launch_bounds__(256) void k_zero_u64(long cap, const int* __restric
 }
 
 void launch_fold_fixed(hipStream_t st, int j0, int cap, const int* d_count, const int* mapping,
-                       const unsigned long long* src_f, const unsigned long long* src_v,
-                       unsigned long long* dst_f, unsigned long long* dst_v) {
+                       int fs, int vs, const unsigned long long* src_f,
+                       const unsigned long long* src_v, unsigned long long* dst_f,
+                       unsigned long long* dst_v) {
   if (cap <= j0 || !mapping) return;
-  hipLaunchKernelGGL(k_fold_fixed, dim3((cap - j0 + 255) / 256), dim3(256), 0, st, j0, cap, d_count,
-                     mapping, src_f, src_v, dst_f, dst_v);
+  const int per = src_v ? 16 : 64;
+  hipLaunchKernelGGL(src_v ? k_fold_fixed<16> : k_fold_fixed<4>, dim3((cap - j0 + per - 1) / per),
+                     dim3(256), 0, st, j0, cap, d_count, mapping, fs, vs, src_f, src_v, dst_f,
+                     dst_v);
   DPAMD_LAUNCH_CHECK();
 }
 
@@ -373,13 +379,14 @@ int finalize_ev_blocks(int ntarget, int nloc, int nbucket) {
 }
 
 void launch_finalize_ev(hipStream_t st, int ntarget, int nloc, int nbucket, int nsec,
-                        const int* type, const double* cpsec, const unsigned long long* facc,
+                        const int* type, const double* cpsec, int fs, int vs,
+                        const unsigned long long* facc,
                         const unsigned long long* vacc, const double* e_bucket, double* force,
                         double* atom_virial, double* partials, double* out10, double* energy,
                         double* virial) {
   const int nparts = finalize_ev_blocks(ntarget, nloc, nbucket);
   hipLaunchKernelGGL(k_finalize_ev, dim3(nparts), dim3(256), 0, st, ntarget, nloc, nbucket, nsec,
-                     type, cpsec, facc, vacc, e_bucket, force, atom_virial, partials);
+                     type, cpsec, fs, vs, facc, vacc, e_bucket, force, atom_virial, partials);
   DPAMD_LAUNCH_CHECK();
   hipLaunchKernelGGL(k_reduce_ev2, dim3(1), dim3(256), 0, st, nparts, partials, out10, energy,
                      virial);

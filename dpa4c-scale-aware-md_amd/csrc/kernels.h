@@ -64,8 +64,8 @@ struct EmbArgs {
   // Backward outputs. Each slot's edge gradient goes to its centre's
   // section sums cpsec [nloc][ntypes][12] (force 3, frame virial 9, fp64)
   // and, in fixed point (fixed.h), to its neighbour's extended-atom slot j:
-  // facc [nall][3] and, when non-null, vacc [nall][9] (launch_fold_fixed
-  // then moves ghost sums onto their owners). The forward clears both sums
+  // facc [nall][fs] (three used) and, when non-null, vacc [nall][vs] (nine
+  // used) (launch_fold_fixed then moves ghost sums onto their owners). The forward clears both sums
   // at its end for the backward: zero_n atoms, or *zero_count when
   // zero_count is non-null.
   // edge_grad [nloc][nnei][3] is written only when non-null (kept for
@@ -73,6 +73,7 @@ struct EmbArgs {
   double* edge_grad;
   unsigned long long* facc;
   unsigned long long* vacc;
+  int fs, vs;
   double* cpsec;
   long zero_n;
   const int* zero_count;
@@ -97,6 +98,47 @@ struct EmbArgs {
   // k < ipw, so its weights are staged in LDS once for WAVES * ipw items
   int ipw;
 };
+
+// Embedding stage with the nets expanded in one variable (expand.hip): T and
+// the edge gradients straight from the neighbour list. The neighbour-side and
+// clearing members are as in EmbArgs.
+struct ExpandArgs {
+  int ntypes, nnei;
+  int emb[3];
+  int sel[kMaxTypes];
+  int sec[kMaxTypes + 1];
+  int type_off[kMaxTypes + 1];
+  int wave_off[kMaxTypes + 1];  // first wave (four centres each) of each centre type
+  unsigned char blocks[kMaxPairs];  // 16-term blocks of each pair's expansion
+  double rcut, rcut_smth, inv_sw, inv_nnei, fix_gmax;
+  const double* envp;     // [npair][8] davg[4], dstd[4]
+  const double* cf;       // [npair][cf_stride], cb [npair][cb_stride]: coefficients
+  const double* cb;       // in the forward's and the backward's operand order
+  long cf_stride, cb_stride;
+  const double* phi_pad;  // [64 H] basis values of a padded slot
+  const double* nets;     // [npair][net_stride] nets as in the model file (fp64)
+  long net_stride;
+  const double* ext;
+  const int* nlist;
+  const int* nreal;
+  const int* items;
+  void* Tt;               // forward out, [L3][ldt] (float in mixed mode, as dT)
+  long ldt;
+  const void* dT;         // backward in [nloc][4][L3]
+  double* edge_grad;
+  // fixed-point sums of the neighbour side: without atom virials facc
+  // [nall][4] (three used), with them facc [nall][16] (force in 0..2, virial
+  // in 4..12) and vacc = facc + 4, so that the values of one edge lie in one
+  // 32- or 128-byte line
+  unsigned long long* facc;
+  unsigned long long* vacc;
+  double* cpart;          // [nloc][12] each centre's own force and frame virial
+  long zero_n;
+  const int* zero_count;
+  int* status;
+};
+void launch_expand_fwd(hipStream_t, const ExpandArgs&, int H, bool f32);
+void launch_expand_bwd(hipStream_t, const ExpandArgs&, int H, bool f32);
 
 struct DescArgs {
   int ntypes, nloc, L3, axis, nnei;
@@ -263,18 +305,18 @@ void launch_rev_count(hipStream_t, long nedge, int nnei, const int* nlist, const
                       int* count, int* rank);
 void launch_rev_fill(hipStream_t, long nedge, int nnei, const int* nlist, const int* mapping,
                      const int* off, const int* rank, int* rev);
-// Fixed-point sums src of extended atoms j in [j0, n) added onto their
-// owners mapping[j] in dst (integer atomics: order-independent); dst may be
+// Fixed-point sums src of extended atoms j in [j0, n) (force [.][fs], virial
+// [.][vs] or null, in src as in dst) added onto their owners mapping[j] in dst (integer atomics: order-independent); dst may be
 // src when every owner lies below j0. n = *d_count when d_count is given (a
 // count on the device, at most cap), else cap; src_v / dst_v may be null.
 void launch_fold_fixed(hipStream_t, int j0, int cap, const int* d_count, const int* mapping,
-                       const unsigned long long* src_f, const unsigned long long* src_v,
+                       int fs, int vs, const unsigned long long* src_f, const unsigned long long* src_v,
                        unsigned long long* dst_f, unsigned long long* dst_v);
 // p[0 .. per * n) = 0 for 64-bit words, n = *d_count (at most cap) or cap
 void launch_zero_u64(hipStream_t, long cap, const int* d_count, int per, unsigned long long* p);
 // se_e2_a: forces, atom virials, energy and frame virial from the
 // embedding backward's section sums cpsec [nloc][nsec][12] and the
-// fixed-point target sums facc [ntarget][3], vacc [ntarget][9] (or null);
+// fixed-point target sums facc [ntarget][fs], vacc [ntarget][vs] (or null);
 // type [nloc]: centres of a negative type have no sections. Per block of 256
 // indices the bucket energies e_bucket [nbucket] and the centres' frame
 // virials are summed into partials [finalize_ev_blocks(...)][10], then added
@@ -282,7 +324,7 @@ void launch_zero_u64(hipStream_t, long cap, const int* d_count, int per, unsigne
 // virial when given).
 int finalize_ev_blocks(int ntarget, int nloc, int nbucket);
 void launch_finalize_ev(hipStream_t, int ntarget, int nloc, int nbucket, int nsec, const int* type,
-                        const double* cpsec, const unsigned long long* facc,
+                        const double* cpsec, int fs, int vs, const unsigned long long* facc,
                         const unsigned long long* vacc, const double* e_bucket, double* force,
                         double* atom_virial, double* partials, double* out10, double* energy,
                         double* virial);

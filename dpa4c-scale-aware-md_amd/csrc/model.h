@@ -50,6 +50,17 @@ void pack_embedding_bf16(const ModelHost& m, const EmbLayout& e, std::vector<flo
 void pack_gemm_bf16(const double* W, int rows, int cols, bool trans, std::vector<uint16_t>& out,
                     bool tile_major = false);
 
+// The embedding nets' expansion (expand.h), in the kernels' operand orders.
+struct ExpandHost {
+  int H = 0;                   // terms are held in H groups of 64
+  std::vector<int> blocks;     // [npair] 16-term blocks in use
+  std::vector<double> fwd, bwd;
+  std::vector<double> phi_pad; // [64 H] basis values of a padded slot
+};
+// False when some net needs more than kExpandMaxTerms terms (or has
+// parameters that are not finite): the nets are then evaluated slot by slot.
+bool build_expansion(const ModelHost& m, ExpandHost& e);
+
 // Offsets (in doubles) of each fitting layer inside a type's block.
 struct FitOffsets {
   long W[3], b[3], idt[3], Wo, bo;

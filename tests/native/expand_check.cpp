@@ -1,0 +1,114 @@
+// The embedding nets' expansion on the host (csrc/expand.cpp): for each model
+// file named on the command line, prints one line
+//   ok H max|G - sum C phi| max|G' - sum C phi'| max|G|
+// over distances from the range's end to the cutoff, with the coefficients
+// read back from both operand layouts, the basis evaluated in fp64 as the
+// kernels do and the net and its tangent in extended precision; or "none"
+// when some net has no short enough expansion.
+#include <cmath>
+#include <cstdio>
+#include <fstream>
+#include <iterator>
+
+#include "../../dpa4c-scale-aware-md_amd/csrc/expand.h"
+#include "../../dpa4c-scale-aware-md_amd/csrc/model.h"
+
+using namespace dpamd;
+namespace dpamd {
+bool emb_supported(int, int, int) { return true; }
+}  // namespace dpamd
+using ld = long double;
+
+int main(int argc, char** argv) {
+  for (int q = 1; q < argc; ++q) {
+    std::ifstream in(argv[q], std::ios::binary);
+    const std::vector<unsigned char> buf((std::istreambuf_iterator<char>(in)), {});
+    ModelHost m;
+    if (!parse_model(buf.data(), buf.size(), m).empty()) return 1;
+    ExpandHost e;
+    if (!build_expansion(m, e)) {
+      std::printf("none\n");
+      continue;
+    }
+    const int np = m.ntypes * m.ntypes, F = m.emb[2], N = 64 * e.H;
+    const int NU2 = expand_nu2(F), NQ2 = expand_nq2(F);
+    double eg = 0, ed = 0, gm = 0;
+    int layouts = 0;
+    for (int p = 0; p < np; ++p) {
+      const double* cf = e.fwd.data() + p * expand_fwd_stride(e.H, F);
+      const double* cb = e.bwd.data() + p * expand_bwd_stride(e.H, F);
+      std::vector<double> C((size_t)N * F);
+      for (int k = 0; k < N; ++k)
+        for (int f = 0; f < F; ++f) {
+          const double v = cf[(((k / 4) * NU2 + f / 32) * 64 + 16 * (k % 4) + f % 16) * 2 + f / 16 % 2];
+          const double w = cb[(((k / 16) * NQ2 + f / 8) * 64 + 16 * (f % 8 / 2) + k % 16) * 2 + f % 2];
+          layouts += v != w || (k >= 16 * e.blocks[p] && v != 0.0);
+          C[(size_t)k * F + f] = v;
+        }
+      const double avg = m.davg[4 * p], sd = m.dstd[4 * p];
+      for (int s = 0; s <= 200; ++s) {
+        const double y = s / 200.0;  // rmin sw / r: 0 at the cutoff, 1 at the range's end
+        // fp64 basis
+        const double iv = 1.0 / (1.0 + y), x = kExpandA * 2.0 * y * iv - kExpandB;
+        std::vector<double> T(N), D(N);
+        auto cheb = [&](int n, double* v, double* d) {
+          double a = 1, b = x, da = 0, db = 1;  // T_0, T_1 and slopes
+          if (n == 0) { *v = 1; *d = 0; return; }
+          for (int k = 1; k < n; ++k) {
+            const double c = 2 * x * b - a, dc = 2 * b + 2 * x * db - da;
+            a = b; b = c; da = db; db = dc;
+          }
+          *v = b; *d = db;
+        };
+        for (int k = 0; k < N; ++k) {
+          const int part[4] = {k / 64 * 64, k / 16 % 4 * 16, k / 4 % 4 * 4, k % 4};
+          double v = 1, d = 0;
+          for (int n : part) {
+            double t, dt;
+            cheb(n, &t, &dt);
+            d = d * t + v * dt;
+            v *= t;
+          }
+          T[k] = v;
+          D[k] = d;
+        }
+        // the net and its slope in extended precision
+        std::vector<ld> h{((ld)y / (ld)kExpandRmin - avg) / sd}, t{1};
+        const double* P = m.emb_params.data() + (size_t)p * m.emb_block;
+        const int L[4] = {1, m.emb[0], m.emb[1], m.emb[2]};
+        for (int k = 0; k < 3; ++k) {
+          std::vector<ld> z(L[k + 1]), zt(L[k + 1]);
+          for (int f = 0; f < L[k + 1]; ++f) {
+            ld a = P[L[k] * L[k + 1] + f], at = 0;
+            for (int c = 0; c < L[k]; ++c) {
+              a += h[c] * P[c * L[k + 1] + f];
+              at += t[c] * P[c * L[k + 1] + f];
+            }
+            z[f] = std::tanh(a);
+            zt[f] = (1 - z[f] * z[f]) * at;
+            if (k > 0 && L[k + 1] == 2 * L[k]) {
+              z[f] += h[f % L[k]];
+              zt[f] += t[f % L[k]];
+            }
+          }
+          P += L[k] * L[k + 1] + L[k + 1];
+          h = z;
+          t = zt;
+        }
+        const double dxds = kExpandA * 2.0 * iv * iv * kExpandRmin * sd;
+        for (int f = 0; f < F; ++f) {
+          double g = 0, d = 0;
+          for (int k = 0; k < N; ++k) {
+            g += C[(size_t)k * F + f] * T[k];
+            d += C[(size_t)k * F + f] * D[k];
+          }
+          eg = std::fmax(eg, std::fabs((double)(g - h[f])));
+          ed = std::fmax(ed, std::fabs((double)(d * dxds - t[f])));
+          gm = std::fmax(gm, std::fabs((double)h[f]));
+        }
+      }
+    }
+    std::printf("ok %d %.3e %.3e %.3e %d\n", e.H, eg, ed, gm, layouts);
+  }
+  return 0;
+}

@@ -1,0 +1,57 @@
+"""The embedding nets' expansion as the host builds it (csrc/expand.cpp),
+without a GPU: accuracy of the values and slopes over the whole range, both
+operand layouts, and the nets that have none."""
+import os
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+
+from _pkg import PKG_DIR, ROOT
+
+HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+
+
+def scaled(dp, kind, scale):
+    """A seeded model whose first-layer weights are scaled: the nets vary
+    `scale` times as fast with the distance."""
+    m = dp.model.random_model(kind, seed=1000)
+    m["emb_params"] = m["emb_params"].copy()
+    m["emb_params"][:, :m["emb"][0]] *= scale
+    return m
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not found")
+def test_expansion_accuracy(dp, tmp_path):
+    exe = str(tmp_path / "expand_check")
+    csrc = os.path.join(PKG_DIR, "csrc")
+    subprocess.run([HIPCC, "-O2", "-std=c++17", "--offload-arch=gfx950", "-w",
+                    os.path.join(ROOT, "tests", "native", "expand_check.cpp"),
+                    os.path.join(csrc, "expand.cpp"), os.path.join(csrc, "model.cpp"), "-o", exe],
+                   check=True)
+    bad = dp.model.random_model("cu", seed=1000)
+    bad["emb_params"] = bad["emb_params"].copy()
+    bad["emb_params"][0, 3] = np.nan
+    cases = [("water", 0.25, 1), ("cu", 1.0, 1), ("water", 1.0, 2), ("hea", 1.0, 2),
+             ("water", 2.5, 4), ("water", 30.0, 0), (bad, None, 0)]
+    paths = []
+    for k, (kind, scale, _) in enumerate(cases):
+        m = kind if scale is None else scaled(dp, kind, scale)
+        paths.append(dp.model.write_model(str(tmp_path / f"m{k}.bin"), m))
+    out = subprocess.run([exe] + paths, check=True, capture_output=True, text=True).stdout
+    lines = out.strip().splitlines()
+    assert len(lines) == len(cases), out
+    for (kind, scale, groups), line in zip(cases, lines):
+        f = line.split()
+        if groups == 0:
+            assert f == ["none"], (kind, scale, line)
+            continue
+        assert f[0] == "ok" and int(f[1]) == groups, (kind, scale, line)
+        eg, ed, gm = (float(v) for v in f[2:5])
+        # values: a sum of 64 groups terms of size <= |G|, each rounded to
+        # 2^-53 a few times; slopes: factors up to (term index) times the
+        # slope in x near the ends, in units where x spans the range
+        assert eg <= 64 * groups * 2.0 ** -53 * gm, line
+        assert ed <= (64 * groups) ** 2 * 2.0 ** -53 * gm * max(scale, 1.0) / 4, line
+        assert f[5] == "0", line
