@@ -46,6 +46,14 @@ struct Buf {
   size_t cap = 0;
 };
 
+// Atoms up to which the fitting stage takes the few-atoms kernels (fit_few.hip):
+// their time grows with the atoms of all types together, that of the general
+// chains with the launches per type. Queued steps, few / general kernels, us:
+// fp64 Cu 256 atoms 178 / 250, 864 262 / 271, 2916 503 / 375; water 192 180 /
+// 285, 1536 323 / 336, 3000 499 / 384; HEA 1024 303 / 431, 3456 639 / 569.
+// Mixed HEA 250 204 / 525, 2662 423 / 586, 5488 687 / 685.
+int few_rows(int types, bool f32) { return f32 ? 1200 * types : 300 + 600 * types; }
+
 enum Stage {
   kStGeom = 0,
   kStNlist,
@@ -93,9 +101,11 @@ struct dp_model {
   double* d_exp_b = nullptr;
   double* d_exp_pad = nullptr;
   double* d_nets = nullptr;
-  // fp64: the first fitting layer's weights of every type transposed,
-  // [nt][F0][L3 axis] (the fused dE/dD -> dE/dT kernel's operand), or null
-  double* d_w0t = nullptr;
+  // the fitting layers' weights of every type transposed ([out][in], at the
+  // layer's offset in the type's block of fit_t_stride): the input gradients'
+  // operand
+  void* d_fit_t = nullptr;
+  size_t fit_t_stride = 0;
   // mixed precision: per type and fitting layer, byte offsets into d_fitf of
   // the pre-split W (forward) and W^T (backward) fragments, -1 if absent
   void* d_fitf = nullptr;
@@ -413,6 +423,117 @@ void expand_args(const dp_model* M, const EmbArgs& ea, ExpandArgs& xa) {
   xa.status = ea.status;
 }
 
+// The fitting stage of more than few_rows() atoms: per centre type the GEMM
+// chain of fitting.hip, the types' chains concurrent on streams of their own.
+template <class E>
+void fit_types(dp_model* M, hipStream_t st, int nb, int Fmax, bool d_from_t, bool fused_ddt,
+               const E* D, const E* Tt, E* dD, E* dT, E* fitb, double* e_bucket, const int* items) {
+  constexpr bool f32 = sizeof(E) == 4;
+  const ModelHost& m = M->host;
+  const int nt = m.ntypes, L3 = m.emb[2], Dn = L3 * m.axis;
+  int active = 0;
+  size_t ws_need = 0, ws_off = 0, ddt_need = 0, ddt_off = 0;
+  for (int t = 0; t < nt; ++t) {
+    const int rows = M->type_off[t + 1] - M->type_off[t];
+    active += rows > 0;
+    const int sp = rows > 0 ? fit_splits(rows, m.fit[0], Dn, M->ncu) : 1;
+    if (sp > 1) ws_need += (size_t)sp * rows * m.fit[0];
+    const int ds = (fused_ddt && rows > 0) ? ddt_splits(rows, L3, M->ncu) : 1;
+    if (ds > 1) ddt_need += (size_t)(ds + 1) * rows * 64;
+  }
+  // the fused input-gradient kernel's split partials, one region per type
+  double* ddt_ws = ddt_need ? need<double>(M, M->ddt_ws, ddt_need) : nullptr;
+  // split-K slices of the first layer, one region per type (the chains run
+  // concurrently)
+  E* split_ws = ws_need ? need<E>(M, M->split_ws, ws_need) : nullptr;
+  const bool fork = active > 1 && !M->arena_on;
+  // With the plain dE/dD product (few rows per type) the type with the most
+  // rows stays on the evaluation stream, enqueued last, and only the others
+  // wait for the fork event (water-12k 1.95 -> 1.91 ms/step); with the fused
+  // kernel every type runs on a stream of its own (keeping one on the
+  // evaluation stream measured 0.3-0.7 % slower on HEA-128k and water-393k).
+  int tmain = -1;
+  if (fork && !fused_ddt) {
+    tmain = 0;
+    for (int t = 1; t < nt; ++t)
+      if (M->type_off[t + 1] - M->type_off[t] > M->type_off[tmain + 1] - M->type_off[tmain])
+        tmain = t;
+  }
+  if (fork) {
+    if (!M->fork_ev) DPAMD_HIP(hipEventCreateWithFlags(&M->fork_ev, hipEventDisableTiming));
+    DPAMD_HIP(hipEventRecord(M->fork_ev, st));
+  }
+  for (int q = 0; q < nt; ++q) {
+    // visiting order: every type but tmain, then tmain
+    const int t = tmain < 0 ? q : (q < tmain ? q : (q + 1 < nt ? q + 1 : tmain));
+    const int rows = M->type_off[t + 1] - M->type_off[t];
+    if (rows <= 0) continue;
+    const bool side = fork && t != tmain;
+    hipStream_t fst = st;
+    if (side) {
+      if (!M->fit_st[t]) {
+        DPAMD_HIP(hipStreamCreateWithFlags(&M->fit_st[t], hipStreamNonBlocking));
+        DPAMD_HIP(hipEventCreateWithFlags(&M->join_ev[t], hipEventDisableTiming));
+      }
+      fst = M->fit_st[t];
+      DPAMD_HIP(hipStreamWaitEvent(fst, M->fork_ev, 0));
+    }
+    const E* P = static_cast<const E*>(M->d_fit) + (size_t)t * m.fit_block;
+    FitNet<E> net{};
+    const int ins[3] = {Dn, m.fit[0], m.fit[1]};
+    for (int k = 0; k < 3; ++k) {
+      net.L[k].W = P + M->fo.W[k];
+      net.L[k].b = P + M->fo.b[k];
+      net.L[k].idt = M->fo.idt[k] >= 0 ? P + M->fo.idt[k] : nullptr;
+      net.L[k].in = ins[k];
+      net.L[k].out = m.fit[k];
+      if (f32 && M->d_fitf) {
+        const char* fb = static_cast<const char*>(M->d_fitf);
+        net.L[k].Wf = M->fitf_off[t][k][0] >= 0 ? fb + M->fitf_off[t][k][0] : nullptr;
+        net.L[k].WfT = M->fitf_off[t][k][1] >= 0 ? fb + M->fitf_off[t][k][1] : nullptr;
+      }
+    }
+    net.Wo = P + M->fo.Wo;
+    net.bo = m.fit_params[(size_t)t * m.fit_block + M->fo.bo];
+    net.bias = m.bias[t];
+    const size_t r0 = (size_t)M->type_off[t];
+    const size_t slab = (size_t)std::max(nb, 1) * Fmax;
+    FitBufs<E> fb{};
+    fb.split = fit_splits(rows, m.fit[0], Dn, M->ncu);
+    if (fb.split > 1) fb.ws = split_ws + ws_off;
+    ws_off += (size_t)fb.split * rows * m.fit[0];
+    E* base = fitb;
+    E** slots[6] = {&fb.H0, &fb.T1, &fb.H1, &fb.dZa, &fb.dZb, &fb.dH};
+    // slab q holds [rows][F] of every type back to back; F <= Fmax. Slab 6
+    // holds the head's partial energies (at most F2 / 16 doubles per row).
+    for (int q = 0; q < 6; ++q) *slots[q] = base + q * slab + r0 * (size_t)Fmax;
+    fb.epart = reinterpret_cast<double*>(base + 6 * slab) + r0 * (size_t)(m.fit[2] / 16);
+    FitDdt ddt{};
+    if (fused_ddt) {
+      if constexpr (f32)
+        ddt.W0T = static_cast<const char*>(M->d_fitf) + M->fitf_off[t][0][1];
+      else
+        ddt.W0T = static_cast<const double*>(M->d_fit_t) + (size_t)t * M->fit_t_stride;
+      ddt.items = items;
+      ddt.pos0 = (int)r0;
+      ddt.dT = dT;
+      ddt.dD = dD ? dD + r0 * Dn : nullptr;
+      ddt.ncu = M->ncu;
+      ddt.nsplit = ddt_splits(rows, L3, M->ncu);
+      ddt.ws = ddt.nsplit > 1 ? ddt_ws + ddt_off : nullptr;
+      if (ddt.nsplit > 1) ddt_off += (size_t)(ddt.nsplit + 1) * rows * 64;
+    }
+    launch_fitting(fst, net, rows, d_from_t ? nullptr : D + r0 * Dn,
+                   d_from_t ? Tt + r0 * 4 : nullptr, 4L * nb, L3, fb, dD ? dD + r0 * Dn : nullptr,
+                   e_bucket + r0, fused_ddt ? &ddt : nullptr);
+    if (side) DPAMD_HIP(hipEventRecord(M->join_ev[t], fst));
+  }
+  if (fork)
+    for (int t = 0; t < nt; ++t)
+      if (t != tmain && M->type_off[t + 1] > M->type_off[t])
+        DPAMD_HIP(hipStreamWaitEvent(st, M->join_ev[t], 0));
+}
+
 // nall: extended atoms, or (d_nall non-null, standalone path) their
 // capacity with the count itself on the device.
 template <class E>
@@ -446,10 +567,16 @@ void run_model_t(dp_model* M, hipStream_t st, int nloc, int nall, const int* d_n
     const int rows = M->type_off[t + 1] - M->type_off[t];
     if (rows > 0) min_rows = std::min(min_rows, rows);
   }
+  // few atoms in all: every type's chain in one set of latency-bound kernels
+  // (fit_few.hip); dp_debug_fused_rows(0) keeps the general kernels
+  int present = 0;
+  for (int t = 0; t < nt; ++t) present += M->type_off[t + 1] > M->type_off[t];
+  const bool few = d_from_t && nb <= few_rows(present, f32) && M->fused_ddt_rows > 0 &&
+                   few_lds_bytes(nb, m.fit[0], sizeof(E)) <= 64 * 1024;
   const bool fused_ddt =
-      d_from_t && (f32 ? M->fitf_off[0][0][1] >= 0
-                       : M->d_w0t != nullptr && min_rows >= M->fused_ddt_rows);
-  E* dD = (!fused_ddt || M->keep_edge_grad) ? need<E>(M, M->dD, (size_t)std::max(nb, 1) * Dn)
+      d_from_t && !few && (f32 ? M->fitf_off[0][0][1] >= 0
+                       : ddt_supported(m.fit[0], L3, axis) && min_rows >= M->fused_ddt_rows);
+  E* dD = ((!fused_ddt && !few) || M->keep_edge_grad) ? need<E>(M, M->dD, (size_t)std::max(nb, 1) * Dn)
                                             : nullptr;
   E* dT = need<E>(M, M->dT, (size_t)nloc * 4 * L3);
   const int Fmax = std::max(m.fit[0], std::max(m.fit[1], m.fit[2]));
@@ -576,110 +703,51 @@ void run_model_t(dp_model* M, hipStream_t st, int nloc, int nall, const int* d_n
   if ((nt > 1 && !expand) || D) launch_descriptor(st, desc_args(M, Tt, D), f32);
   record(M, st, kStDescr + 1);
 
-  int active = 0;
-  size_t ws_need = 0, ws_off = 0, ddt_need = 0, ddt_off = 0;
-  for (int t = 0; t < nt; ++t) {
-    const int rows = M->type_off[t + 1] - M->type_off[t];
-    active += rows > 0;
-    const int sp = rows > 0 ? fit_splits(rows, m.fit[0], Dn, M->ncu) : 1;
-    if (sp > 1) ws_need += (size_t)sp * rows * m.fit[0];
-    const int ds = (fused_ddt && rows > 0) ? ddt_splits(rows, L3, M->ncu) : 1;
-    if (ds > 1) ddt_need += (size_t)(ds + 1) * rows * 64;
-  }
-  // the fused input-gradient kernel's split partials, one region per type
-  double* ddt_ws = ddt_need ? need<double>(M, M->ddt_ws, ddt_need) : nullptr;
-  // split-K slices of the first layer, one region per type (the chains run
-  // concurrently)
-  E* split_ws = ws_need ? need<E>(M, M->split_ws, ws_need) : nullptr;
-  const bool fork = active > 1 && !M->arena_on;
-  // With the plain dE/dD product (few rows per type) the type with the most
-  // rows stays on the evaluation stream, enqueued last, and only the others
-  // wait for the fork event (water-12k 1.95 -> 1.91 ms/step); with the fused
-  // kernel every type runs on a stream of its own (keeping one on the
-  // evaluation stream measured 0.3-0.7 % slower on HEA-128k and water-393k).
-  int tmain = -1;
-  if (fork && !fused_ddt) {
-    tmain = 0;
-    for (int t = 1; t < nt; ++t)
-      if (M->type_off[t + 1] - M->type_off[t] > M->type_off[tmain + 1] - M->type_off[tmain])
-        tmain = t;
-  }
-  if (fork) {
-    if (!M->fork_ev) DPAMD_HIP(hipEventCreateWithFlags(&M->fork_ev, hipEventDisableTiming));
-    DPAMD_HIP(hipEventRecord(M->fork_ev, st));
-  }
-  for (int q = 0; q < nt; ++q) {
-    // visiting order: every type but tmain, then tmain
-    const int t = tmain < 0 ? q : (q < tmain ? q : (q + 1 < nt ? q + 1 : tmain));
-    const int rows = M->type_off[t + 1] - M->type_off[t];
-    if (rows <= 0) continue;
-    const bool side = fork && t != tmain;
-    hipStream_t fst = st;
-    if (side) {
-      if (!M->fit_st[t]) {
-        DPAMD_HIP(hipStreamCreateWithFlags(&M->fit_st[t], hipStreamNonBlocking));
-        DPAMD_HIP(hipEventCreateWithFlags(&M->join_ev[t], hipEventDisableTiming));
+  if (few) {
+    FewArgs<E> fa{};
+    fa.nt = nt;
+    fa.nb = nb;
+    fa.L3 = L3;
+    for (int k = 0; k < 3; ++k) fa.F[k] = m.fit[k];
+    fa.tile_rows = few_tile_rows(nb);
+    fa.slices = few_slices(L3);
+    int tiles = 0;
+    for (int t = 0; t < nt; ++t) {
+      const E* P = static_cast<const E*>(M->d_fit) + (size_t)t * m.fit_block;
+      const E* PT = static_cast<const E*>(M->d_fit_t) + (size_t)t * M->fit_t_stride;
+      FewNet<E>& net = fa.net[t];
+      for (int k = 0; k < 3; ++k) {
+        net.W[k] = P + M->fo.W[k];
+        net.WT[k] = PT + M->fo.W[k];
+        net.b[k] = P + M->fo.b[k];
+        net.idt[k] = M->fo.idt[k] >= 0 ? P + M->fo.idt[k] : nullptr;
       }
-      fst = M->fit_st[t];
-      DPAMD_HIP(hipStreamWaitEvent(fst, M->fork_ev, 0));
+      net.Wo = P + M->fo.Wo;
+      net.bo = m.fit_params[(size_t)t * m.fit_block + M->fo.bo];
+      net.bias = m.bias[t];
+      net.pos0 = M->type_off[t];
+      net.rows = M->type_off[t + 1] - M->type_off[t];
+      net.tile0 = tiles;
+      tiles += (net.rows + fa.tile_rows - 1) / fa.tile_rows;
     }
-    const E* P = static_cast<const E*>(M->d_fit) + (size_t)t * m.fit_block;
-    FitNet<E> net{};
-    const int ins[3] = {Dn, m.fit[0], m.fit[1]};
-    for (int k = 0; k < 3; ++k) {
-      net.L[k].W = P + M->fo.W[k];
-      net.L[k].b = P + M->fo.b[k];
-      net.L[k].idt = M->fo.idt[k] >= 0 ? P + M->fo.idt[k] : nullptr;
-      net.L[k].in = ins[k];
-      net.L[k].out = m.fit[k];
-      if (f32 && M->d_fitf) {
-        const char* fb = static_cast<const char*>(M->d_fitf);
-        net.L[k].Wf = M->fitf_off[t][k][0] >= 0 ? fb + M->fitf_off[t][k][0] : nullptr;
-        net.L[k].WfT = M->fitf_off[t][k][1] >= 0 ? fb + M->fitf_off[t][k][1] : nullptr;
-      }
-    }
-    net.Wo = P + M->fo.Wo;
-    net.bo = m.fit_params[(size_t)t * m.fit_block + M->fo.bo];
-    net.bias = m.bias[t];
-    const size_t r0 = (size_t)M->type_off[t];
+    fa.Tt = Tt;
+    fa.ldt = 4L * nb;
+    E** slots[6] = {&fa.H0, &fa.T1, &fa.H1, &fa.dZa, &fa.dZb, &fa.dH};
     const size_t slab = (size_t)std::max(nb, 1) * Fmax;
-    FitBufs<E> fb{};
-    fb.split = fit_splits(rows, m.fit[0], Dn, M->ncu);
-    if (fb.split > 1) fb.ws = split_ws + ws_off;
-    ws_off += (size_t)fb.split * rows * m.fit[0];
-    E* base = fitb;
-    E** slots[6] = {&fb.H0, &fb.T1, &fb.H1, &fb.dZa, &fb.dZb, &fb.dH};
-    // slab q holds [rows][F] of every type back to back; F <= Fmax. Slab 6
-    // holds the head's partial energies (at most F2 / 16 doubles per row).
-    for (int q = 0; q < 6; ++q) *slots[q] = base + q * slab + r0 * (size_t)Fmax;
-    fb.epart = reinterpret_cast<double*>(base + 6 * slab) + r0 * (size_t)(m.fit[2] / 16);
-    FitDdt ddt{};
-    if (fused_ddt) {
-      if constexpr (f32)
-        ddt.W0T = static_cast<const char*>(M->d_fitf) + M->fitf_off[t][0][1];
-      else
-        ddt.W0T = M->d_w0t + (size_t)t * m.fit[0] * Dn;
-      ddt.items = items;
-      ddt.pos0 = (int)r0;
-      ddt.dT = dT;
-      ddt.dD = dD ? dD + r0 * Dn : nullptr;
-      ddt.ncu = M->ncu;
-      ddt.nsplit = ddt_splits(rows, L3, M->ncu);
-      ddt.ws = ddt.nsplit > 1 ? ddt_ws + ddt_off : nullptr;
-      if (ddt.nsplit > 1) ddt_off += (size_t)(ddt.nsplit + 1) * rows * 64;
-    }
-    launch_fitting(fst, net, rows, d_from_t ? nullptr : D + r0 * Dn,
-                   d_from_t ? Tt + r0 * 4 : nullptr, 4L * nb, L3, fb, dD ? dD + r0 * Dn : nullptr,
-                   e_bucket + r0, fused_ddt ? &ddt : nullptr);
-    if (side) DPAMD_HIP(hipEventRecord(M->join_ev[t], fst));
+    for (int q = 0; q < 6; ++q) *slots[q] = fitb + q * slab;
+    fa.epart = reinterpret_cast<double*>(fitb + 6 * slab);
+    fa.e = e_bucket;
+    fa.ws = need<double>(M, M->ddt_ws, (size_t)(fa.slices + 1) * std::max(nb, 1) * 64);
+    fa.items = items;
+    fa.dT = dT;
+    fa.dD = dD;
+    launch_fitting_few(st, fa);
+  } else {
+    fit_types<E>(M, st, nb, Fmax, d_from_t, fused_ddt, D, Tt, dD, dT, fitb, e_bucket, items);
   }
-  if (fork)
-    for (int t = 0; t < nt; ++t)
-      if (t != tmain && M->type_off[t + 1] > M->type_off[t])
-        DPAMD_HIP(hipStreamWaitEvent(st, M->join_ev[t], 0));
   record(M, st, kStFit + 1);
 
-  if (!fused_ddt) launch_dT(st, nb, L3, axis, items, Tt, dD, dT);
+  if (!fused_ddt && !few) launch_dT(st, nb, L3, axis, items, Tt, dD, dT);
   M->dd_valid = dD != nullptr;
   record(M, st, kStDT + 1);
 
@@ -1414,20 +1482,30 @@ int dp_create(const char* path, int gpu_rank, const void* file_content, size_t c
     } else {
       upload(M->d_emb, emb);
       upload(M->d_fit, m.fit_params);
-      const int Dn = m.emb[2] * m.axis, F0 = m.fit[0];
-      if (ddt_supported(F0, m.emb[2], m.axis)) {
-        const FitOffsets fo = fit_offsets(m);
-        std::vector<double> w0t((size_t)m.ntypes * F0 * Dn);
-        for (int t = 0; t < m.ntypes; ++t) {
-          const double* W = m.fit_params.data() + (size_t)t * m.fit_block + fo.W[0];
-          for (int n = 0; n < Dn; ++n)
-            for (int k = 0; k < F0; ++k) w0t[((size_t)t * F0 + k) * Dn + n] = W[(size_t)n * F0 + k];
-        }
-        upload(M->d_w0t, w0t);
-      }
+    }
+    M->fo = fit_offsets(m);
+    {
+      const int ins[3] = {m.emb[2] * m.axis, m.fit[0], m.fit[1]};
+      M->fit_t_stride = ((size_t)m.fit_block + 15) / 16 * 16;  // (16-byte aligned blocks)
+      auto transposed = [&](auto zero) {
+        std::vector<decltype(zero)> out(m.ntypes * M->fit_t_stride, zero);
+        for (int t = 0; t < m.ntypes; ++t)
+          for (int k = 0; k < 3; ++k) {
+            const double* W = m.fit_params.data() + (size_t)t * m.fit_block + M->fo.W[k];
+            auto* o = out.data() + t * M->fit_t_stride + M->fo.W[k];
+            const int in = ins[k], on = m.fit[k];
+            for (int i0 = 0; i0 < in; i0 += 32)
+              for (int j0 = 0; j0 < on; j0 += 32)
+                for (int j = j0; j < std::min(on, j0 + 32); ++j)
+                  for (int i = i0; i < std::min(in, i0 + 32); ++i)
+                    o[(size_t)j * in + i] = (decltype(zero))W[(size_t)i * on + j];
+          }
+        return out;
+      };
+      if (mixed) upload(M->d_fit_t, transposed(0.0f));
+      else upload(M->d_fit_t, transposed(0.0));
     }
     M->bytes_peak = M->bytes_now;
-    M->fo = fit_offsets(m);
     if (const char* g = std::getenv("DPAMD_GRAPH")) M->graph_on = std::atoi(g) != 0;
   });
   if (rc != DP_OK) {
@@ -1446,7 +1524,7 @@ void dp_destroy(dp_model* M) {
   for (Buf* b : M->bufs)
     if (b->p) (void)hipFree(b->p);
   for (void* p : {M->d_emb, static_cast<void*>(M->d_envp), static_cast<void*>(M->d_tpad), M->d_fit,
-                  M->d_fitf, M->d_c4, static_cast<void*>(M->d_w0t), static_cast<void*>(M->d_exp_f),
+                  M->d_fitf, M->d_c4, M->d_fit_t, static_cast<void*>(M->d_exp_f),
                   static_cast<void*>(M->d_exp_b), static_cast<void*>(M->d_exp_pad),
                   static_cast<void*>(M->d_nets)})
     if (p) (void)hipFree(p);

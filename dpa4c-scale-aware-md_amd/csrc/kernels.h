@@ -293,6 +293,36 @@ template <class T>
 void launch_fitting(hipStream_t, const FitNet<T>&, int rows, const T* D, const T* Tt, long ldt,
                     int L3, const FitBufs<T>&, T* dD, double* e_bucket,
                     const FitDdt* ddt = nullptr);
+// Few atoms (fit_few.hip): the whole fitting stage of every type, dE/dT
+// included. Activations [nb][F] in bucket order; ws: (few_slices(L3) + 1) nb 64
+// doubles.
+template <class T>
+struct FewNet {
+  const T *W[3], *WT[3], *b[3], *idt[3], *Wo;  // WT: W transposed
+  double bo, bias;
+  int rows, pos0;  // rows of the type, bucket position of the first
+  int tile0;       // first row tile in the launches' grid
+};
+template <class T>
+struct FewArgs {
+  int nt, nb, L3;
+  int tile_rows;  // few_tile_rows(nb)
+  int slices;     // few_slices(L3)
+  int F[3];
+  FewNet<T> net[kMaxTypes];
+  const T* Tt;
+  long ldt;
+  T *H0, *T1, *H1, *dZa, *dZb, *dH;
+  double *epart, *e, *ws;
+  const int* items;
+  T* dT;
+  T* dD;  // [nb][16 L3] when kept for inspection, else null
+};
+int few_slices(int L3);
+int few_tile_rows(int nb);
+size_t few_lds_bytes(int nb, int F0, size_t esize);  // at most 64 KB
+template <class T>
+void launch_fitting_few(hipStream_t, const FewArgs<T>&);
 // Tt column-major in bucket order (element (pos, a, m) at Tt[a * 4 nloc +
 // 4 pos + m]), dT in atom order (items maps bucket position to atom).
 template <class T>

@@ -98,8 +98,9 @@ enum {
  * `precision` DP_PREC_MODEL takes the precision recorded in the model file
  * (upstream, the evaluation precision is a property of the trained model);
  * DP_PREC_FP64 evaluates everything in fp64; DP_PREC_MIXED
- * evaluates the embedding nets, the descriptor and the fitting net in fp32
- * (FP32 MFMA) and the env matrix, edge gradients, forces, virials and energy
+ * evaluates the descriptor and the fitting net in fp32 (and the embedding
+ * nets, when they are evaluated slot by slot; their expansion is summed in
+ * fp64) and the env matrix, edge gradients, forces, virials and energy
  * sums in fp64 -- the reference's mixed-precision rule (fp32
  * embedding/fitting, fp64 env matrix, force and virial accumulation), checked
  * against its acceptance limits (data/numeric-tolerances.json:3-9).
@@ -309,7 +310,9 @@ int dp_debug_keep(dp_model* model, int keep);
  * kernel (dE/dD never stored) when every atom type has at least `rows` atoms
  * (default 12288; 0: always), and otherwise as the plain product
  * dE/dD = dZ0 W0^T followed by a separate dE/dT pass, which is faster for
- * few atoms per type. Both forms give the same results to rounding. No
+ * few atoms per type. Systems of a few hundred to a few thousand atoms in all
+ * run a set of kernels of their own (both precisions); rows == 0 switches
+ * those off too. All forms give the same results to rounding. No
  * counterpart in the reference: a parity-test hook, so that both forms are
  * checked at the sizes the oracle evaluates. */
 int dp_debug_fused_rows(dp_model* model, int rows);
