@@ -5,10 +5,11 @@
 // unless some net of the model has no short enough expansion; embed.hip and
 // embed_f32.hip then evaluate the nets slot by slot.
 //
-// Work unit: one wave (a block of its own: nothing is shared, so blocks of
-// one wave leave no barrier and no tail) owns four consecutive centres of one
-// type; lane group g (lane = 16 g + c) walks the slots of centre g, 16 at a
-// time. A round prepares 64 slots, one a lane (environment row, basis
+// Work unit: one wave (W = 1: a block of its own, nothing is shared, so there
+// is no barrier and no tail) owns four consecutive centres of one type; lane
+// group g (lane = 16 g + c) walks the slots of centre g, 16 at a time. Systems
+// with too few centres to fill the device give the four centres to a block of
+// W = 4 waves that share out the rounds and the products' tiles. A round prepares 64 slots, one a lane (environment row, basis
 // values), in LDS; the products then read them per centre.
 //
 // Forward, per neighbour section: M[(m, b)][(p, l)] += R[m] T_16b (x) T_4p T_l
@@ -115,6 +116,13 @@ __device__ __forceinline__ double inv_1p(double y) {
   return fma(fma(-w, v, 1.0), v, v);
 }
 
+// LDS written by the block's waves made visible to them (W = 1: to the wave)
+template <int W>
+__device__ __forceinline__ void block_sync() {
+  if constexpr (W > 1) __syncthreads();
+  else wave_lds_sync();
+}
+
 // sum over the 16 lanes of a lane group, in every lane
 __device__ __forceinline__ double sum_c16(double v) {
 #pragma unroll
@@ -215,16 +223,19 @@ constexpr int fwd_lds(int H) {
   return rec > m ? rec : m;
 }
 constexpr int bwd_lds(int H) { return 64 * kRecB(H); }
-static_assert(bwd_lds(1) >= 16 * kTr, "transposition buffer fits the records");
+static_assert(bwd_lds(1) >= 16 * kTr, "transposition buffer fits a wave's records");
 static_assert(fwd_lds(1) >= 2 * (32 + 64) && bwd_lds(1) >= 2 * (32 + 64), "net_at scratch");
 
 }  // namespace
 
-template <class E, int NU3, int H>
-__global__ __launch_bounds__(64, H > 2 ? 1 : 2) void k_expand_fwd(ExpandArgs a) {
-  extern __shared__ __align__(16) double lds[];
+template <class E, int NU3, int H, int W>
+__global__ __launch_bounds__(64 * W, H > 2 ? 1 : 2) void k_expand_fwd(ExpandArgs a) {
+  extern __shared__ __align__(16) double lds_all[];
   constexpr int RS = kRecF(H), LD = 64 * H + 4, NU2 = (NU3 + 1) / 2;
-  const int lane = threadIdx.x, g = lane >> 4, c = lane & 15;
+  constexpr int NT = (NU3 + W - 1) / W;  // T tiles of a wave: u = W k + w
+  const int w = W > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+  double* lds = lds_all + w * fwd_lds(H);
   const Centres q4 = my_centres(a, g);
   const int ti = q4.ti, L3 = a.emb[2];
   const double xi = a.ext[3L * q4.i], yi = a.ext[3L * q4.i + 1], zi = a.ext[3L * q4.i + 2];
@@ -233,9 +244,9 @@ __global__ __launch_bounds__(64, H > 2 ? 1 : 2) void k_expand_fwd(ExpandArgs a) 
   const int eL = c & 3, eP = (c >> 2) ? 3 + (c >> 2) : 0, eB = (c & 3) ? 6 + (c & 3) : 0;
   const int eR = 10 + (c >> 2);
   double* rec = lds + lane * RS;
-  d4 T[NU3];
+  d4 T[NT];
 #pragma unroll
-  for (int u = 0; u < NU3; ++u) T[u] = d4{0.0, 0.0, 0.0, 0.0};
+  for (int u = 0; u < NT; ++u) T[u] = d4{0.0, 0.0, 0.0, 0.0};
   bool close = false;  // some slot of this lane is outside the expansion
 
   for (int tj = 0; tj < a.ntypes; ++tj) {
@@ -261,21 +272,22 @@ __global__ __launch_bounds__(64, H > 2 ? 1 : 2) void k_expand_fwd(ExpandArgs a) 
       const double pp = a.phi_pad[64 * h + lane];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const double w = (double)(a.sel[tj] - nrj[j]) * pp;
+        const double np = w == 0 ? (double)(a.sel[tj] - nrj[j]) * pp : 0.0;
 #pragma unroll
-        for (int m = 0; m < 4; ++m) acc[j][h][m] = w * (-avg[m] * isd[m]);
+        for (int m = 0; m < 4; ++m) acc[j][h][m] = np * (-avg[m] * isd[m]);
       }
     }
-    // coordinates one tile ahead, indices two (clamped into the section)
+    // coordinates one round ahead, indices two (clamped into the section)
     double nx = 0.0, ny = 0.0, nz = 0.0;
-    if (c < nr) {
-      const long j = row[c];
+    const int s0 = 16 * w + c;
+    if (s0 < nr) {
+      const long j = row[s0];
       nx = a.ext[3 * j];
       ny = a.ext[3 * j + 1];
       nz = a.ext[3 * j + 2];
     }
-    int jn = row[min(16 + c, slast)];
-    for (int t = 0; t < most; t += 16) {
+    int jn = row[min(s0 + 16 * W, slast)];
+    for (int t = 16 * w; t < most; t += 16 * W) {
       const int slot = t + c;
       double Rn[4] = {0.0, 0.0, 0.0, 0.0}, x = 0.0;
       if (slot < nr) {
@@ -287,12 +299,12 @@ __global__ __launch_bounds__(64, H > 2 ? 1 : 2) void k_expand_fwd(ExpandArgs a) 
           Rn[0] = Rn[1] = Rn[2] = Rn[3] = 0.0;
         }
       }
-      if (slot + 16 < nr) {
+      if (slot + 16 * W < nr) {
         nx = a.ext[3L * jn];
         ny = a.ext[3L * jn + 1];
         nz = a.ext[3L * jn + 2];
       }
-      jn = row[min(slot + 32, slast)];
+      jn = row[min(slot + 32 * W, slast)];
       double v[kNumBasis<H>];
       basis_values<H>(x, v);
       wave_lds_sync();
@@ -324,35 +336,64 @@ __global__ __launch_bounds__(64, H > 2 ? 1 : 2) void k_expand_fwd(ExpandArgs a) 
       for (int h = 0; h < H; ++h)
 #pragma unroll
         for (int m = 0; m < 4; ++m) lds[(4 * m + j) * LD + 64 * h + lane] = acc[j][h][m];
-    wave_lds_sync();
-    const double2* C = reinterpret_cast<const double2*>(a.cf) + (long)pair * (a.cf_stride / 2) + lane;
-    const double* A = lds + c * LD + g;
     const int nq = 4 * nblk;
-    double2 b0[NU2], b1[NU2];
+    if constexpr (W == 1) {
+      wave_lds_sync();
+      const double2* C = reinterpret_cast<const double2*>(a.cf) + (long)pair * (a.cf_stride / 2) + lane;
+      const double* A = lds + c * LD + g;
+      double2 b0[NU2], b1[NU2];
 #pragma unroll
-    for (int u = 0; u < NU2; ++u) {
-      b0[u] = C[64 * u];
-      b1[u] = C[64 * (NU2 + u)];
-    }
-    for (int q = 0; q < nq; q += 2) {
-      const double a0 = A[4 * q], a1 = A[4 * q + 4];
-      const double2* Cn = C + 64L * NU2 * min(q + 2, nq - 2);
+      for (int u = 0; u < NU2; ++u) {
+        b0[u] = C[64 * u];
+        b1[u] = C[64 * (NU2 + u)];
+      }
+      for (int q = 0; q < nq; q += 2) {
+        const double a0 = A[4 * q], a1 = A[4 * q + 4];
+        const double2* Cn = C + 64L * NU2 * min(q + 2, nq - 2);
 #pragma unroll
-      for (int u = 0; u < NU3; ++u) T[u] = mfma_f64(a0, u & 1 ? b0[u / 2].y : b0[u / 2].x, T[u]);
+        for (int u = 0; u < NU3; ++u) T[u] = mfma_f64(a0, u & 1 ? b0[u / 2].y : b0[u / 2].x, T[u]);
 #pragma unroll
-      for (int u = 0; u < NU2; ++u) b0[u] = Cn[64 * u];
+        for (int u = 0; u < NU2; ++u) b0[u] = Cn[64 * u];
 #pragma unroll
-      for (int u = 0; u < NU3; ++u) T[u] = mfma_f64(a1, u & 1 ? b1[u / 2].y : b1[u / 2].x, T[u]);
+        for (int u = 0; u < NU3; ++u) T[u] = mfma_f64(a1, u & 1 ? b1[u / 2].y : b1[u / 2].x, T[u]);
 #pragma unroll
-      for (int u = 0; u < NU2; ++u) b1[u] = Cn[64 * (NU2 + u)];
+        for (int u = 0; u < NU2; ++u) b1[u] = Cn[64 * (NU2 + u)];
+      }
+    } else {
+      // the waves' shares of M are added where they are read; each wave its
+      // tiles u = W k + w of T, four k-steps' coefficients in flight
+      __syncthreads();
+      const double* A = lds_all + c * LD + g;
+      const double* C = a.cf + (long)pair * a.cf_stride + 2 * lane;
+      for (int q = 0; q < nq; q += 4) {
+        double av[4], b[4][NT];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int k = 0; k < NT; ++k) {
+            const int u = min(W * k + w, NU3 - 1);
+            b[e][k] = C[128L * (NU2 * (q + e) + u / 2) + (u & 1)];
+          }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          av[e] = A[4 * (q + e)];
+#pragma unroll
+          for (int v = 1; v < W; ++v) av[e] += A[v * fwd_lds(H) + 4 * (q + e)];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int k = 0; k < NT; ++k) T[k] = mfma_f64(av[e], b[e][k], T[k]);
+      }
+      __syncthreads();
     }
   }
   // lane (g, c): T of centre g (bucket position pos0 + g), features 16u + c
   E* Tt = static_cast<E*>(a.Tt) + 4L * (q4.pos0 + g);
   if (q4.ok) {
 #pragma unroll
-    for (int u = 0; u < NU3; ++u) {
-      const int f = 16 * u + c;
+    for (int u = 0; u < NT; ++u) {
+      const int f = 16 * (W * u + w) + c;
       if (f < L3) {
         Vec4<E> o;
         o.x = (E)(T[u][0] * a.inv_nnei);
@@ -364,9 +405,14 @@ __global__ __launch_bounds__(64, H > 2 ? 1 : 2) void k_expand_fwd(ExpandArgs a) 
     }
   }
   // slots outside the expansion's range (rare): the net itself, added to the
-  // centre's T, which this wave alone writes
-  if (__builtin_expect(__ballot(close) != 0, 0)) {
+  // centre's T, which this block alone writes
+  bool any = __ballot(close) != 0;
+  if constexpr (W > 1) any = __syncthreads_or(any);
+  if (__builtin_expect(any, 0)) {
     __threadfence();
+    if constexpr (W > 1) __syncthreads();
+  }
+  if (__builtin_expect(any && w == 0, 0)) {
     for (int j = 0; j < 4; ++j) {
       const int i = lane_int(q4.i, 16 * j);
       const double x0 = lane_double(xi, 16 * j), y0 = lane_double(yi, 16 * j),
@@ -413,7 +459,7 @@ __global__ __launch_bounds__(64, H > 2 ? 1 : 2) void k_expand_fwd(ExpandArgs a) 
   }
   // the backward's fixed-point sums, cleared as the blocks end
   const long n = a.zero_count ? (long)*a.zero_count : a.zero_n;
-  const long stride = (long)gridDim.x * 64, q0 = (long)blockIdx.x * 64 + lane;
+  const long stride = (long)gridDim.x * (64 * W), q0 = (long)blockIdx.x * (64 * W) + threadIdx.x;
   const long words = (a.vacc ? 16 : 4) * n;
   for (long q = q0; q < words; q += stride) a.facc[q] = 0ull;
 }
@@ -463,12 +509,14 @@ __device__ __forceinline__ void scatter_records(const ExpandArgs& a, const doubl
 }
 }  // namespace
 
-template <class E, int NU3, int H, bool AV>
-__global__ __launch_bounds__(64, H > 2 ? 1 : 2) void k_expand_bwd(ExpandArgs a) {
-  extern __shared__ __align__(16) double lds[];
+template <class E, int NU3, int H, bool AV, int W>
+__global__ __launch_bounds__(64 * W, H > 2 ? 1 : 2) void k_expand_bwd(ExpandArgs a) {
+  extern __shared__ __align__(16) double lds_all[];
   constexpr int RB = kRecB(H);
   constexpr int NQ2 = NU3 == 8 ? 16 : 13;  // expand_nq2(L3)
-  const int lane = threadIdx.x, g = lane >> 4, c = lane & 15;
+  const int w = W > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+  double* lds = lds_all + w * bwd_lds(H);
   const Centres q4 = my_centres(a, g);
   const int ti = q4.ti, L3 = a.emb[2];
   const double xi = a.ext[3L * q4.i], yi = a.ext[3L * q4.i + 1], zi = a.ext[3L * q4.i + 2];
@@ -491,7 +539,7 @@ __global__ __launch_bounds__(64, H > 2 ? 1 : 2) void k_expand_bwd(ExpandArgs a) 
 #pragma unroll
     for (int j = 0; j < 4; ++j) nrj[j] = lane_int(nr, 16 * j);
     const int most = max(max(nrj[0], nrj[1]), max(nrj[2], nrj[3]));
-    if (a.edge_grad && q4.ok)
+    if (a.edge_grad && q4.ok && w == 0)
       for (int s = nr + c; s <= slast; s += 16)
         for (int q = 0; q < 3; ++q) a.edge_grad[3 * (ebase + s) + q] = 0.0;
     if (most == 0) continue;
@@ -516,44 +564,47 @@ __global__ __launch_bounds__(64, H > 2 ? 1 : 2) void k_expand_bwd(ExpandArgs a) 
       const double2* C = reinterpret_cast<const double2*>(a.cb) + (long)pair * (a.cb_stride / 2) + lane;
 #pragma unroll
       for (int h = 0; h < H; ++h) {
-        wave_lds_sync();
-        for (int b = 0; b < 4; ++b) {
+        block_sync<W>();
+        // (W = 4: wave w forms term block w)
+        for (int b = w; b < 4; b += W) {
           d4 acc = d4{0.0, 0.0, 0.0, 0.0};
           if (4 * h + b < nblk) {
             const double2* Cb = C + 64L * NQ2 * (4 * h + b);
             d4 acc1 = d4{0.0, 0.0, 0.0, 0.0};
-            double2 w[NQ2];
+            double2 cv[NQ2];
 #pragma unroll
-            for (int q = 0; q < NQ2; ++q) w[q] = Cb[64 * q];
+            for (int q = 0; q < NQ2; ++q) cv[q] = Cb[64 * q];
 #pragma unroll
             for (int q = 0; q < NQ2; ++q) {
-              acc = mfma_f64(dTa[2 * q], w[q].x, acc);
-              acc1 = mfma_f64(dTa[2 * q + 1], w[q].y, acc1);
+              acc = mfma_f64(dTa[2 * q], cv[q].x, acc);
+              acc1 = mfma_f64(dTa[2 * q + 1], cv[q].y, acc1);
             }
             acc += acc1;
           }
           // lane (g, c): centre g, term 16b + c, register m
 #pragma unroll
-          for (int m = 0; m < 4; ++m) lds[(4 * g + m) * kTr + 16 * b + c] = acc[m];
+          for (int m = 0; m < 4; ++m) lds_all[(4 * g + m) * kTr + 16 * b + c] = acc[m];
         }
-        wave_lds_sync();
+        block_sync<W>();
         // A operand of centre j: row c = 4m + b, k = 4q + g
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
           for (int q = 0; q < 4; ++q)
-            dMa[j][h][q] = lds[(4 * j + (c >> 2)) * kTr + 16 * (c & 3) + 4 * q + g];
+            dMa[j][h][q] = lds_all[(4 * j + (c >> 2)) * kTr + 16 * (c & 3) + 4 * q + g];
       }
     }
+    if constexpr (W > 1) __syncthreads();  // the records overlay the transposition buffer
     double nx = 0.0, ny = 0.0, nz = 0.0;
-    int jc = row[min(c, slast)];
-    if (c < nr) {
+    const int s0 = 16 * w + c;
+    int jc = row[min(s0, slast)];
+    if (s0 < nr) {
       nx = a.ext[3L * jc];
       ny = a.ext[3L * jc + 1];
       nz = a.ext[3L * jc + 2];
     }
-    int jn = row[min(16 + c, slast)];
-    for (int t = 0; t < most; t += 16) {
+    int jn = row[min(s0 + 16 * W, slast)];
+    for (int t = 16 * w; t < most; t += 16 * W) {
       const int slot = t + c;
       bool live = slot < nr;
       const double d[3] = {nx - xi, ny - yi, nz - zi};
@@ -571,12 +622,12 @@ __global__ __launch_bounds__(64, H > 2 ? 1 : 2) void k_expand_bwd(ExpandArgs a) 
         }
       }
       jc = jn;
-      if (slot + 16 < nr) {
+      if (slot + 16 * W < nr) {
         nx = a.ext[3L * jn];
         ny = a.ext[3L * jn + 1];
         nz = a.ext[3L * jn + 2];
       }
-      jn = row[min(slot + 32, slast)];
+      jn = row[min(slot + 32 * W, slast)];
       double v[kNumBasis<H>], s[kNumBasis<H>];
       basis_values<H>(x, v);
       basis_slopes<H>(x, v, s);
@@ -630,11 +681,11 @@ __global__ __launch_bounds__(64, H > 2 ? 1 : 2) void k_expand_bwd(ExpandArgs a) 
 #pragma unroll
         for (int h = 1; h < H; ++h) {
           const double2 ph = *reinterpret_cast<const double2*>(r + 22 + 2 * h);
-          const double w = pb.x * ph.x, wd = fma(pb.y, ph.x, pb.x * ph.y);
+          const double wh = pb.x * ph.x, wd = fma(pb.y, ph.x, pb.x * ph.y);
 #pragma unroll
           for (int m = 0; m < 4; ++m) {
-            u[m] = fma(w, Y[h][m], u[m]);
-            vs = fma(R[m], fma(wd, Y[h][m], w * Yd[h][m]), vs);
+            u[m] = fma(wh, Y[h][m], u[m]);
+            vs = fma(R[m], fma(wd, Y[h][m], wh * Yd[h][m]), vs);
           }
         }
 #pragma unroll
@@ -662,7 +713,9 @@ __global__ __launch_bounds__(64, H > 2 ? 1 : 2) void k_expand_bwd(ExpandArgs a) 
     }
   }
   // slots outside the expansion's range (rare): the net and its slope
-  if (__builtin_expect(__ballot(close) != 0, 0)) {
+  bool any = __ballot(close) != 0;
+  if constexpr (W > 1) any = __syncthreads_or(any);
+  if (__builtin_expect(any && w == 0, 0)) {
     for (int j = 0; j < 4; ++j) {
       const int i = lane_int(q4.i, 16 * j);
       const double x0 = lane_double(xi, 16 * j), y0 = lane_double(yi, 16 * j),
@@ -703,9 +756,9 @@ __global__ __launch_bounds__(64, H > 2 ? 1 : 2) void k_expand_bwd(ExpandArgs a) 
               for (int e = 0; e < 2; ++e) {
                 const int f = lane + 64 * e;
                 if (f >= L3) continue;
-                const double w = (double)dTi[m * L3 + f];
-                u = fma(w, G[e], u);
-                vs = fma(R[m] * w, dG[e], vs);
+                const double dt = (double)dTi[m * L3 + f];
+                u = fma(dt, G[e], u);
+                vs = fma(R[m] * dt, dG[e], vs);
               }
               nd[m] = add_xor32(add_xor16(sum_c16(u))) * a.inv_nnei;
             }
@@ -732,7 +785,19 @@ __global__ __launch_bounds__(64, H > 2 ? 1 : 2) void k_expand_bwd(ExpandArgs a) 
   // the centre's own sums over the 16 lanes of its group
 #pragma unroll
   for (int q = 0; q < 12; ++q) own[q] = sum_c16(own[q]);
-  if (q4.ok && c == 0) {
+  if constexpr (W > 1) {
+    // ... and over the block's waves, in order
+    __syncthreads();
+    if (c == 0)
+#pragma unroll
+      for (int q = 0; q < 12; ++q) lds_all[(w * 4 + g) * 12 + q] = own[q];
+    __syncthreads();
+    if (w == 0 && c == 0)
+#pragma unroll
+      for (int q = 0; q < 12; ++q)
+        for (int v = 1; v < W; ++v) own[q] += lds_all[(v * 4 + g) * 12 + q];
+  }
+  if (q4.ok && c == 0 && w == 0) {
     double* o = a.cpart + 12L * q4.i;
 #pragma unroll
     for (int q = 0; q < 12; ++q) o[q] = own[q];
@@ -740,28 +805,33 @@ __global__ __launch_bounds__(64, H > 2 ? 1 : 2) void k_expand_bwd(ExpandArgs a) 
 }
 
 namespace {
-template <class E, int NU3, int H>
-void launch_fwd(hipStream_t st, const ExpandArgs& a, int nwave) {
-  hipLaunchKernelGGL((k_expand_fwd<E, NU3, H>), dim3(nwave), dim3(64),
-                     sizeof(double) * fwd_lds(H), st, a);
+// Blocks of four waves up to this many groups of four centres (half a group
+// per SIMD). Queued steps with blocks of one / four waves, us: water 192 atoms
+// 177 / 147, 1536 338 / 314, 3993 440 / 442, 12288 861 / 975; Cu 864 262 / 236,
+// 4000 461 / 462; HEA mixed 1024 262 / 232, 3456 489 / 528.
+constexpr int kSharedGroups = 512;
+
+template <class K>
+void run(K kern, hipStream_t st, const ExpandArgs& a, int nblock, int waves, size_t bytes) {
+  DPAMD_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)bytes));
+  hipLaunchKernelGGL(kern, dim3(nblock), dim3(64 * waves), bytes, st, a);
+}
+template <class E, int NU3, int H, int W>
+void launch_w(hipStream_t st, const ExpandArgs& a, int nblock, bool bwd) {
+  if (!bwd) run(k_expand_fwd<E, NU3, H, W>, st, a, nblock, W, sizeof(double) * W * fwd_lds(H));
+  else if (a.vacc) run(k_expand_bwd<E, NU3, H, true, W>, st, a, nblock, W, sizeof(double) * W * bwd_lds(H));
+  else run(k_expand_bwd<E, NU3, H, false, W>, st, a, nblock, W, sizeof(double) * W * bwd_lds(H));
 }
 template <class E, int NU3, int H>
-void launch_bwd(hipStream_t st, const ExpandArgs& a, int nwave) {
-  const size_t bytes = sizeof(double) * bwd_lds(H);
-  if (a.vacc)
-    hipLaunchKernelGGL((k_expand_bwd<E, NU3, H, true>), dim3(nwave), dim3(64), bytes, st, a);
-  else
-    hipLaunchKernelGGL((k_expand_bwd<E, NU3, H, false>), dim3(nwave), dim3(64), bytes, st, a);
+void launch_g(hipStream_t st, const ExpandArgs& a, int ngroup, bool bwd) {
+  if (ngroup <= kSharedGroups) launch_w<E, NU3, H, 4>(st, a, ngroup, bwd);
+  else launch_w<E, NU3, H, 1>(st, a, ngroup, bwd);
 }
 template <class E, int NU3>
-void launch_h(hipStream_t st, const ExpandArgs& a, int H, int nwave, bool bwd) {
-  if (bwd) {
-    H == 1 ? launch_bwd<E, NU3, 1>(st, a, nwave)
-           : H == 2 ? launch_bwd<E, NU3, 2>(st, a, nwave) : launch_bwd<E, NU3, 4>(st, a, nwave);
-  } else {
-    H == 1 ? launch_fwd<E, NU3, 1>(st, a, nwave)
-           : H == 2 ? launch_fwd<E, NU3, 2>(st, a, nwave) : launch_fwd<E, NU3, 4>(st, a, nwave);
-  }
+void launch_h(hipStream_t st, const ExpandArgs& a, int H, int ngroup, bool bwd) {
+  H == 1 ? launch_g<E, NU3, 1>(st, a, ngroup, bwd)
+         : H == 2 ? launch_g<E, NU3, 2>(st, a, ngroup, bwd) : launch_g<E, NU3, 4>(st, a, ngroup, bwd);
   DPAMD_LAUNCH_CHECK();
 }
 void launch_expand(hipStream_t st, const ExpandArgs& a, int H, bool f32, bool bwd) {

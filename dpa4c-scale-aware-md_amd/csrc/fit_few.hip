@@ -40,19 +40,42 @@ __device__ __forceinline__ Tile find_tile(const FewArgs<T>& a, int block) {
   return Tile{t, row0, a.net[t].rows, (long)a.net[t].pos0 + row0};
 }
 
+// A tile's accumulator: fp64, or fp32 partial sums of at most 64 products
+// added up in fp64 (flush), which leaves no more rounding than the bf16
+// three-piece products of the general kernels (whose fp32 accumulators run
+// over all of K): without it the forces of small mixed systems were 12 % further
+// from their fp64 values than with those.
+template <class T>
+struct TileAcc {
+  d4 s = d4{0.0, 0.0, 0.0, 0.0};
+  __device__ __forceinline__ void add(double a, double b) { s = mfma(a, b, s); }
+  __device__ __forceinline__ void flush() {}
+};
+template <>
+struct TileAcc<float> {
+  d4 s = d4{0.0, 0.0, 0.0, 0.0};
+  f4 part = f4{0.0f, 0.0f, 0.0f, 0.0f};
+  __device__ __forceinline__ void add(float a, float b) { part = mfma(a, b, part); }
+  __device__ __forceinline__ void flush() {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) s[r] += (double)part[r];
+    part = f4{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+};
+
 // The waves' partial tiles (RT times 16 rows x 16 columns) in LDS; element
 // (row, col) is then their sum in wave order.
 template <class T, int RT>
-__device__ __forceinline__ void park(T (*red)[16 * RT][17], const typename Frag<T>::V (&acc)[RT],
-                                     int w, int g, int c) {
+__device__ __forceinline__ void park(double (*red)[16 * RT][17], const TileAcc<T> (&acc)[RT], int w,
+                                     int g, int c) {
 #pragma unroll
   for (int t = 0; t < RT; ++t)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) red[w][16 * t + Frag<T>::row(g, r)][c] = acc[t][r];
+    for (int r = 0; r < 4; ++r) red[w][16 * t + Frag<T>::row(g, r)][c] = acc[t].s[r];
   __syncthreads();
 }
 template <class T, int NW, int RT>
-__device__ __forceinline__ T sum_waves(T (*red)[16 * RT][17], int row, int col, T bias = T(0)) {
+__device__ __forceinline__ T sum_waves(double (*red)[16 * RT][17], int row, int col, T bias = T(0)) {
   double s = red[0][row][col];
 #pragma unroll
   for (int k = 1; k < NW; ++k) s += red[k][row][col];
@@ -68,7 +91,7 @@ __device__ __forceinline__ float act(float x) { return tanh_f32(x); }
 constexpr int kFirstWaves = 8;
 template <class T, int RT>
 __global__ __launch_bounds__(64 * kFirstWaves) void k_few_first(FewArgs<T> a) {
-  __shared__ T red[kFirstWaves][16 * RT][17];
+  __shared__ double red[kFirstWaves][16 * RT][17];
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
   const Tile tl = find_tile(a, blockIdx.y);
   const FewNet<T>& net = a.net[tl.t];
@@ -86,9 +109,7 @@ __global__ __launch_bounds__(64 * kFirstWaves) void k_few_first(FewArgs<T> a) {
   const int per = (a.L3 + kFirstWaves - 1) / kFirstWaves;
   const int a0 = w * per, a1 = min(a.L3, a0 + per);
   const T* W = net.W[0] + (long)g * N + col0 + c;
-  typename Frag<T>::V acc[RT];
-#pragma unroll
-  for (int t = 0; t < RT; ++t) acc[t] = typename Frag<T>::V{0, 0, 0, 0};
+  TileAcc<T> acc[RT];
   constexpr int U = RT > 1 ? 2 : 4;  // columns a (four k-steps each) in flight
   for (int k = a0; k < a1; k += U) {
     Vec4<T> ta[U][RT];
@@ -109,9 +130,11 @@ __global__ __launch_bounds__(64 * kFirstWaves) void k_few_first(FewArgs<T> a) {
 #pragma unroll
         for (int t = 0; t < RT; ++t) {
           const Vec4<T>&x = ta[u][t], &y = tb[t][q];
-          acc[t] = mfma(x.x * y.x + x.y * y.y + x.z * y.z + x.w * y.w, b[u][q], acc[t]);
+          acc[t].add(x.x * y.x + x.y * y.y + x.z * y.z + x.w * y.w, b[u][q]);
         }
     }
+#pragma unroll
+    for (int t = 0; t < RT; ++t) acc[t].flush();
   }
   park<T, RT>(red, acc, w, g, c);
   const int col = col0 + (threadIdx.x & 15);
@@ -129,7 +152,7 @@ __global__ __launch_bounds__(64 * kFirstWaves) void k_few_first(FewArgs<T> a) {
 // (1 - H0^2). ([.]: on square layers.)
 template <class T, int STAGE, int RT>
 __global__ __launch_bounds__(256) void k_few_layer(FewArgs<T> a) {
-  __shared__ T red[4][16 * RT][17];
+  __shared__ double red[4][16 * RT][17];
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
   const Tile tl = find_tile(a, blockIdx.y);
   const FewNet<T>& net = a.net[tl.t];
@@ -166,9 +189,7 @@ __global__ __launch_bounds__(256) void k_few_layer(FewArgs<T> a) {
             : STAGE == 2 ? (net.idt[2] ? a.H1[o] : T(0))
             : STAGE == 3 ? a.T1[o] : a.H0[o];
   }
-  typename Frag<T>::V acc[RT];
-#pragma unroll
-  for (int t = 0; t < RT; ++t) acc[t] = typename Frag<T>::V{0, 0, 0, 0};
+  TileAcc<T> acc[RT];
   for (int q0 = 0; q0 < per; q0 += kU) {
     T av[kU][RT], bv[kU];
 #pragma unroll
@@ -182,7 +203,9 @@ __global__ __launch_bounds__(256) void k_few_layer(FewArgs<T> a) {
     for (int u = 0; u < kU; ++u)
       if (q0 + u < per)
 #pragma unroll
-        for (int t = 0; t < RT; ++t) acc[t] = mfma(av[u][t], bv[u], acc[t]);
+        for (int t = 0; t < RT; ++t) acc[t].add(av[u][t], bv[u]);
+#pragma unroll
+    for (int t = 0; t < RT; ++t) acc[t].flush();
   }
   park<T, RT>(red, acc, w, g, c);
 #pragma unroll
@@ -273,7 +296,7 @@ __global__ __launch_bounds__(256) void k_few_dT(FewArgs<T> a) {
   }
   const T* Zr = Z + c * LD + g;
   const int col0 = kDtCols * blockIdx.x + 2 * w, ncol = min(2, a.L3 - col0);
-  typename Frag<T>::V acc[RT];
+  TileAcc<T> acc[RT];
   Vec4<T> ta[RT];
   // step: kU k-steps of column col0 + step / chunks; W0^T[k][16 col + c]
   const int chunks = (nq + kU - 1) / kU, steps = ncol > 0 ? ncol * chunks : 0;
@@ -289,7 +312,7 @@ __global__ __launch_bounds__(256) void k_few_dT(FewArgs<T> a) {
     if (q0 == 0) {
 #pragma unroll
       for (int t = 0; t < RT; ++t) {
-        acc[t] = typename Frag<T>::V{0, 0, 0, 0};
+        acc[t] = TileAcc<T>{};
         ta[t] = *reinterpret_cast<const Vec4<T>*>(Tr[t] + col * a.ldt);
       }
     }
@@ -310,9 +333,11 @@ __global__ __launch_bounds__(256) void k_few_dT(FewArgs<T> a) {
       for (int u = 0; u < 4; ++u)
         if (q0 + u0 + u < nq)
 #pragma unroll
-          for (int t = 0; t < RT; ++t) acc[t] = mfma(wv[u0 + u], z[(u0 / 4) & 1][u][t], acc[t]);
+          for (int t = 0; t < RT; ++t) acc[t].add(wv[u0 + u], z[(u0 / 4) & 1][u][t]);
       __builtin_amdgcn_sched_barrier(0);
     }
+#pragma unroll
+    for (int t = 0; t < RT; ++t) acc[t].flush();
     if (q0 + kU < nq) return;
 #pragma unroll
     for (int t = 0; t < RT; ++t) {
@@ -324,8 +349,8 @@ __global__ __launch_bounds__(256) void k_few_dT(FewArgs<T> a) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const Vec4<T>& y = tb[t][r];
-          v += (double)acc[t][r] * (double)(m == 0 ? y.x : m == 1 ? y.y : m == 2 ? y.z : y.w);
-          acc2[t][r][m] += acc[t][r] * tm[m];
+          v += acc[t].s[r] * (double)(m == 0 ? y.x : m == 1 ? y.y : m == 2 ? y.z : y.w);
+          acc2[t][r][m] += (T)acc[t].s[r] * tm[m];
         }
         s[m] = add_xor32(add_xor16(v));
       }
@@ -336,7 +361,7 @@ __global__ __launch_bounds__(256) void k_few_dT(FewArgs<T> a) {
         else a.ws[((long)a.slices * a.nb + pos) * 64 + 16 * g + col] = mine;
         if (a.dD)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) a.dD[pos * Dn + 16 * col + Frag<T>::row(g, r)] = acc[t][r];
+          for (int r = 0; r < 4; ++r) a.dD[pos * Dn + 16 * col + Frag<T>::row(g, r)] = (T)acc[t].s[r];
       }
     }
   };

@@ -53,14 +53,15 @@ def test_both_evaluations(dp, orc, kind, scale, drop, mixed):
 
 
 @pytest.mark.parametrize("mixed", [False, True])
-@pytest.mark.parametrize("kind", ["water", "hea"])
-def test_pairs_closer_than_the_expansion(dp, orc, kind, mixed):
+@pytest.mark.parametrize("kind,cells", [("water", 4), ("hea", 4), ("water", 9), ("hea", 11)])
+def test_pairs_closer_than_the_expansion(dp, orc, kind, cells, mixed):
     """Pairs on both sides of the range's end (0.6 A), several of one centre
-    and of neighbouring centres."""
+    and of neighbouring centres, with four centres to a block of waves and (the
+    larger systems) to a wave."""
     if kind == "water":
-        coord, atype, box = dp.systems.water(4, 12.42, seed=54)
+        coord, atype, box = dp.systems.water(cells, 3.105 * cells, seed=54)
     else:
-        coord, atype, box = dp.systems.bcc_hea(4, 3.2, seed=55)
+        coord, atype, box = dp.systems.bcc_hea(cells, 3.2, seed=55)
     coord = coord.copy()
     n = len(atype)
     for k, (a, b, r) in enumerate([(0, n - 1, 0.59), (0, n // 2, 0.45), (1, n - 2, 0.61), (5, 6, 0.5)]):
