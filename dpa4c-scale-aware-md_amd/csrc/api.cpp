@@ -1344,7 +1344,8 @@ void upload_c4(dp_model* M) {
   const size_t o_temb = put(c.temb.data(), c.temb.size() * 4);
   const size_t o_mean = put(c.mean.data(), c.mean.size() * 4);
   const size_t o_istd = put(c.istd.data(), c.istd.size() * 4);
-  const size_t o_w0t = put(c.w0t.data(), c.w0t.size() * 4);
+  const size_t o_wf = put(c.wf.data(), c.wf.size() * 4);
+  const size_t o_wb = put(c.wb.data(), c.wb.size() * 4);
   const size_t o_b0 = put(c.b0.data(), c.b0.size() * 4);
   const size_t o_wh = put(c.wh.data(), c.wh.size() * 4);
   const size_t o_bias = put(c.bias.data(), c.bias.size() * 8);
@@ -1360,7 +1361,8 @@ void upload_c4(dp_model* M) {
   p.temb = reinterpret_cast<const float*>(base + o_temb);
   p.mean = reinterpret_cast<const float*>(base + o_mean);
   p.istd = reinterpret_cast<const float*>(base + o_istd);
-  p.w0t = reinterpret_cast<const float*>(base + o_w0t);
+  p.wf = reinterpret_cast<const float*>(base + o_wf);
+  p.wb = reinterpret_cast<const float*>(base + o_wb);
   p.b0 = reinterpret_cast<const float*>(base + o_b0);
   p.wh = reinterpret_cast<const float*>(base + o_wh);
   p.bias = reinterpret_cast<const double*>(base + o_bias);

@@ -13,11 +13,11 @@
 //                   accumulates the 40 moments and 2 envelope masses in
 //                   registers, reduced over the group by a butterfly. One
 //                   lane per edge means no geometry is recomputed per channel.
-//   k_c4_node       one thread per node: normalisation, alignment and probe
-//                   projections, the 70 invariants, standardisation, the
-//                   fitting net forward and its input gradient (weights read
-//                   as wave-uniform scalar loads), then the readout VJP down
-//                   to cotangents of the 42 raw sums.
+//   k_c4_node       one wave per 16 or 64 nodes: normalisation, alignment and
+//                   probe projections, the 70 invariants, standardisation,
+//                   the fitting net forward and its input gradient on the
+//                   matrix cores, then the readout VJP down to cotangents of
+//                   the 42 raw sums.
 //   k_c4_edge_grad  G lanes per node recompute each edge and contract it with
 //                   the node's cotangents into dE/dd.
 //   k_c4_edge_force on the standalone path (complete list folded onto
@@ -342,7 +342,7 @@ __global__ __launch_bounds__(kEdgeBlock) void k_c4_moments(C4Params p, Src src, 
   }
 }
 
-// ---- pass 2: readout, fitting, readout VJP (one thread per node) ---------
+// ---- pass 2: readout, fitting, readout VJP --------------------------------
 // packed degree-two components -> symmetric traceless 3x3 (graph_compress.cuh:520-530)
 __device__ __forceinline__ void stf(const float q[5], float M[3][3]) {
   M[0][0] = -q[2] * kInvSq6 + q[4] * kInvSq2;
@@ -455,26 +455,41 @@ __device__ __forceinline__ float act_val(int act, float z, float& dact) {
   return z * sg;
 }
 
-template <class IT>
-__global__ __launch_bounds__(kBlock) void k_c4_node(C4Params p, int nnodes,
-                                                   const IT* __restrict__ type,
-                                                   const float* __restrict__ mom,
-                                                   double* __restrict__ energy,
-                                                   float* __restrict__ cot) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= nnodes) return;
-  const int ti = (int)type[i];
-  f4* co = reinterpret_cast<f4*>(cot + (long)i * kC4Mom);
-  if (ti < 0 || ti >= p.nt) {
-    energy[i] = 0.0;
-#pragma unroll
-    for (int q = 0; q < 11; ++q) co[q] = f4{0.f, 0.f, 0.f, 0.f};
-    return;
-  }
-  float D[kC4Out];
+// One wave takes A atoms (64, or 16 for few of them). The readout and its VJP
+// run one atom a lane (A = 16: the four lane groups repeat them); the fitting
+// layer and its input gradient are products on the matrix cores, transposed so
+// that one's result registers are the other's operand (fp32 16x16x4 MFMA,
+// lane = 16 g + c):
+//   Z'[h][atom] = W0' D'   k-step (t, r): feature 16 t + 4 g + r of atom c, the
+//                          lane's four values of t one 16-byte LDS read;
+//                          register r is hidden unit 16 u + 4 g + r of atom c
+//   dD'[q][atom] = W0 dZ'  k-step (u, r): that hidden unit
+// with the weights packed in the lanes' order (wf, wb: 16 bytes a lane for
+// four k-steps). One thread an atom with the 13.4k FMAs of the layer in a
+// serial loop kept only 32 waves busy at 2,016 atoms and issued every FMA on
+// the VALU at 499,800: 66 us against 15 now, and 337 against 231.
+constexpr int kNodeLd = 84;  // LDS row of one atom's features: 80 + 4 (16-byte reads: distinct banks)
+template <class IT, int A>
+__global__ __launch_bounds__(64, 2) void k_c4_node(C4Params p, int nnodes,
+                                                  const IT* __restrict__ type,
+                                                  const float* __restrict__ mom,
+                                                  double* __restrict__ energy,
+                                                  float* __restrict__ cot) {
+  __shared__ __align__(16) float Ds[A][kNodeLd];
+  const int lane = threadIdx.x, g = lane >> 4, c16 = lane & 15;
+  const int slot = A == 64 ? lane : c16;  // this lane's atom of the wave
+  const int i = (int)blockIdx.x * A + slot;
+  const bool here = i < nnodes;
+  const int ic = here ? i : nnodes - 1;
+  const int t_in = (int)type[ic];
+  const bool valid = t_in >= 0 && t_in < p.nt;
+  const int ti = valid ? t_in : 0;
+  const bool writes = here && (A == 64 || g == 0);
+  float e = 0.f;
   {
+    float D[80];
     float m[kC4Mom];
-    load_mom(mom + (long)i * kC4Mom, m);
+    load_mom(mom + (long)ic * kC4Mom, m);
     Readout R;
     project(p, m, R);
     int o = 0;
@@ -543,38 +558,105 @@ __global__ __launch_bounds__(kBlock) void k_c4_node(C4Params p, int nnodes,
     for (int c = 0; c < 8; ++c) D[o++] = p.temb[ti * 8 + c];
 #pragma unroll
     for (int q = 0; q < kC4Out; ++q) D[q] = (D[q] - p.mean[q]) * p.istd[q];
+#pragma unroll
+    for (int q = kC4Out; q < 80; ++q) D[q] = 0.f;
+    // a square residual layer's share of the energy: D . wh
+    if ((p.resnet & 1) && p.H == kC4Out)
+#pragma unroll
+      for (int q = 0; q < kC4Out; ++q) e = fmaf(p.wh[q], D[q], e);
+    if (A == 64 || g == 0)
+#pragma unroll
+      for (int q = 0; q < 20; ++q)
+        *reinterpret_cast<f4*>(&Ds[slot][4 * q]) = f4{D[4 * q], D[4 * q + 1], D[4 * q + 2], D[4 * q + 3]};
   }
-  // fitting: e = sum_h wh[h] act(D . W0[:, h] + b0[h]) (+ D[h] on a square
-  // residual layer) + bh + bias[type]; dD accumulated in the same pass
-  float dD[kC4Out];
+  wave_lds_sync();
+  // fitting: e = sum_h wh[h] act(D . W0[:, h] + b0[h]) (+ D . wh on a square
+  // residual layer) + bh + bias[type], and dD, 16 hidden units at a time
+  constexpr int NA = A / 16;
+  f4 dDt[NA][5];
+  float ea[NA];
 #pragma unroll
-  for (int q = 0; q < kC4Out; ++q) dD[q] = 0.f;
-  const bool res = (p.resnet & 1) && p.H == kC4Out;
-  float e = 0.f;
-  for (int h = 0; h < p.H; ++h) {
-    const float* w = p.w0t + (long)h * kC4W0Ld;
-    float z = p.b0[h];
+  for (int n = 0; n < NA; ++n) {
+    ea[n] = 0.f;
 #pragma unroll
-    for (int q = 0; q < kC4Out; ++q) z = fmaf(D[q], w[q], z);
-    float da;
-    const float a = act_val(p.act, z, da);
-    const float wh = p.wh[h];
-    e = fmaf(wh, a, e);
-    const float dz = wh * da;
-#pragma unroll
-    for (int q = 0; q < kC4Out; ++q) dD[q] = fmaf(dz, w[q], dD[q]);
+    for (int v = 0; v < 5; ++v) dDt[n][v] = f4{0.f, 0.f, 0.f, 0.f};
   }
-  if (res) {
-    for (int h = 0; h < kC4Out; ++h) e = fmaf(p.wh[h], D[h], e);
+  const f4* wf = reinterpret_cast<const f4*>(p.wf) + lane;
+  const f4* wb = reinterpret_cast<const f4*>(p.wb) + lane;
+  const int nu = (p.H + 15) / 16;
+  f4 fa[5], fb[5];
+#pragma unroll
+  for (int t = 0; t < 5; ++t) fa[t] = wf[64 * t];
+  for (int u = 0; u < nu; ++u) {
+#pragma unroll
+    for (int t = 0; t < 5; ++t) fb[t] = wb[64 * (5 * u + t)];
+    const f4 bias = *reinterpret_cast<const f4*>(p.b0 + 16 * u + 4 * g);
+    const f4 wh = *reinterpret_cast<const f4*>(p.wh + 16 * u + 4 * g);
+    f4 z[NA];
+#pragma unroll
+    for (int n = 0; n < NA; ++n) z[n] = bias;
+#pragma unroll
+    for (int t = 0; t < 5; ++t) {
+      f4 d[NA];
+#pragma unroll
+      for (int n = 0; n < NA; ++n) d[n] = *reinterpret_cast<const f4*>(&Ds[16 * n + c16][16 * t + 4 * g]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int n = 0; n < NA; ++n) z[n] = mfma_f32(fa[t][r], d[n][r], z[n]);
+    }
+    // the next units' forward weights, behind this one's products
+    const int un = min(u + 1, nu - 1);
+#pragma unroll
+    for (int t = 0; t < 5; ++t) fa[t] = wf[64 * (5 * un + t)];
+#pragma unroll
+    for (int n = 0; n < NA; ++n)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float da;
+        const float a = act_val(p.act, z[n][r], da);
+        ea[n] = fmaf(wh[r], a, ea[n]);
+        z[n][r] = wh[r] * da;
+      }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int v = 0; v < 5; ++v)
+#pragma unroll
+        for (int n = 0; n < NA; ++n) dDt[n][v] = mfma_f32(fb[v][r], z[n][r], dDt[n][v]);
+  }
+  // energies: summed over the lane groups; lane (g, c) then holds its tiles'
+  // atoms c, of which A = 64 keeps tile g
+#pragma unroll
+  for (int n = 0; n < NA; ++n) {
+    const float s = add_xor32(add_xor16(ea[n]));
+    if (A == 16 || n == g) e += s;
+  }
+  wave_lds_sync();
+#pragma unroll
+  for (int n = 0; n < NA; ++n)
+#pragma unroll
+    for (int v = 0; v < 5; ++v) *reinterpret_cast<f4*>(&Ds[16 * n + c16][16 * v + 4 * g]) = dDt[n][v];
+  wave_lds_sync();
+  float dD[72];
+#pragma unroll
+  for (int q = 0; q < 18; ++q) {
+    const f4 v = *reinterpret_cast<const f4*>(&Ds[slot][4 * q]);
+    dD[4 * q] = v[0];
+    dD[4 * q + 1] = v[1];
+    dD[4 * q + 2] = v[2];
+    dD[4 * q + 3] = v[3];
+  }
+  if ((p.resnet & 1) && p.H == kC4Out)
 #pragma unroll
     for (int q = 0; q < kC4Out; ++q) dD[q] += p.wh[q];
-  }
-  energy[i] = (double)(e + p.bh) + p.bias[ti];
+  if (writes) energy[i] = valid ? (double)(e + p.bh) + p.bias[ti] : 0.0;
+  f4* co = reinterpret_cast<f4*>(cot + (long)ic * kC4Mom);
   // ---- readout VJP: dD (standardised) -> cotangents of the raw sums ----
 #pragma unroll
   for (int q = 0; q < kC4Out; ++q) dD[q] *= p.istd[q];
   float m[kC4Mom];
-  load_mom(mom + (long)i * kC4Mom, m);
+  load_mom(mom + (long)ic * kC4Mom, m);
   Readout R;
   project(p, m, R);
   float gav[3][4], gat[5][4], gpv[3][4], gpt[5][2], gS[2][3][3];
@@ -734,8 +816,10 @@ __global__ __launch_bounds__(kBlock) void k_c4_node(C4Params p, int nnodes,
   c[kMs] = 0.5f * R.ns * (gdiv0 - g_ns * R.ns * R.ns);
   c[kMa] = 0.5f * R.na * (gdiv1 - g_na * R.na * R.na);
   c[42] = c[43] = 0.f;
+  if (!writes) return;
 #pragma unroll
-  for (int q = 0; q < 11; ++q) co[q] = f4{c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3]};
+  for (int q = 0; q < 11; ++q)
+    co[q] = valid ? f4{c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3]} : f4{0.f, 0.f, 0.f, 0.f};
 }
 
 // ---- pass 3: edge gradients -------------------------------------------------
@@ -1064,20 +1148,36 @@ void launch_c4_moments(hipStream_t st, const C4Params& p, const C4Graph& s, int 
   moments_launch(st, p, GraphSrc{s}, n, mom, status);
 }
 
+namespace {
+// Nodes up to which a wave takes 16 of them. More waves hide the chain of the
+// readout while the chip is not full (whole evaluation, 16 against 64 nodes a
+// wave: 109 to 121 us at 2,016 atoms, 131 to 143 at 8,788, 229 to 236 at
+// 32,000); past that the readout, run four times over with 16, costs more than
+// it hides (388 to 389 at 62,500, 657 to 642 at 131,072, 2,286 to 2,201 at
+// 500,000).
+constexpr int kNodeFew = 32768;
+template <class IT>
+void node_launch(hipStream_t st, const C4Params& p, int n, const IT* type, const float* mom,
+                 double* energy, float* cot) {
+  if (n <= 0) return;
+  if (n <= kNodeFew)
+    hipLaunchKernelGGL((k_c4_node<IT, 16>), dim3((n + 15) / 16), dim3(64), 0, st, p, n, type, mom,
+                       energy, cot);
+  else
+    hipLaunchKernelGGL((k_c4_node<IT, 64>), dim3((n + 63) / 64), dim3(64), 0, st, p, n, type, mom,
+                       energy, cot);
+  DPAMD_LAUNCH_CHECK();
+}
+}  // namespace
+
 void launch_c4_node(hipStream_t st, const C4Params& p, int n, const int* type, const float* mom,
                     double* energy, float* cot) {
-  if (n <= 0) return;
-  hipLaunchKernelGGL(k_c4_node<int>, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, p, n,
-                     type, mom, energy, cot);
-  DPAMD_LAUNCH_CHECK();
+  node_launch(st, p, n, type, mom, energy, cot);
 }
 
 void launch_c4_node(hipStream_t st, const C4Params& p, int n, const long* type, const float* mom,
                     double* energy, float* cot) {
-  if (n <= 0) return;
-  hipLaunchKernelGGL(k_c4_node<long>, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, p, n,
-                     type, mom, energy, cot);
-  DPAMD_LAUNCH_CHECK();
+  node_launch(st, p, n, type, mom, energy, cot);
 }
 
 void launch_c4_edge_grad(hipStream_t st, const C4Params& p, const C4Nlist& s, int n,

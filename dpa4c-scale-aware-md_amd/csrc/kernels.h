@@ -375,7 +375,6 @@ void launch_scatter_energy(hipStream_t, int nloc, const int* items, const double
 // scalar [8], vector [3][4], tensor [5][4], the two envelope masses, 2 pad.
 constexpr int kC4Mom = 44;
 constexpr int kC4Out = 70;   // descriptor width
-constexpr int kC4W0Ld = 72;  // row stride of the transposed first fitting layer
 struct C4Params {
   const float* table;  // [n_int][6][8]: coefficient k of channel c at [i][k][c]
   const float* film;   // [nt*nt][8][2] PairFiLM (scale, shift)
@@ -383,9 +382,13 @@ struct C4Params {
   const float* temb;   // [nt][8] type embedding
   const float* mean;   // [70]
   const float* istd;   // [70]
-  const float* w0t;    // [H][kC4W0Ld] first fitting layer, transposed
-  const float* b0;     // [H]
-  const float* wh;     // [H] head
+  // first fitting layer in the node kernel's operand order, for hidden units
+  // 16 u .. 16 u + 15 (zero past H): wf [u][5 t][64 lanes][4 r] =
+  // W0[16 t + 4 g + r][16 u + c], wb [u][5 v][64][4] = W0[16 v + c][16 u + 4 g + r]
+  const float* wf;
+  const float* wb;
+  const float* b0;     // [H] and wh [H] head, zero-padded to a multiple of 16
+  const float* wh;
   const double* bias;  // [nt] bias_atom_e
   float bh;            // head bias
   int nt, n_int, H, act, resnet;

@@ -348,10 +348,22 @@ std::string parse_c4_model(const unsigned char* buf, size_t len, ModelHost& m, C
   if (!r.ok) return "model file truncated in parameters";
   if (r.off != len) return "trailing bytes in model file";
   c.bh = bh[0];
-  // first layer transposed: row h holds W0[:, h], padded to kC4W0Ld
-  c.w0t.assign((size_t)c.H * kC4W0Ld, 0.f);
-  for (int q = 0; q < kC4Out; ++q)
-    for (int h = 0; h < c.H; ++h) c.w0t[(size_t)h * kC4W0Ld + q] = w0[(size_t)q * c.H + h];
+  // first layer in the node kernel's operand order (C4Params)
+  const int nu = (c.H + 15) / 16;
+  c.wf.assign((size_t)nu * 5 * 256, 0.f);
+  c.wb.assign((size_t)nu * 5 * 256, 0.f);
+  auto w = [&](int q, int h) { return q < kC4Out && h < c.H ? w0[(size_t)q * c.H + h] : 0.f; };
+  for (int u = 0; u < nu; ++u)
+    for (int t = 0; t < 5; ++t)
+      for (int lane = 0; lane < 64; ++lane)
+        for (int r = 0; r < 4; ++r) {
+          const int g = lane >> 4, l = lane & 15;
+          const size_t at = (((size_t)u * 5 + t) * 64 + lane) * 4 + r;
+          c.wf[at] = w(16 * t + 4 * g + r, 16 * u + l);
+          c.wb[at] = w(16 * t + l, 16 * u + 4 * g + r);
+        }
+  c.b0.resize((size_t)16 * nu, 0.f);
+  c.wh.resize((size_t)16 * nu, 0.f);
   return "";
 }
 

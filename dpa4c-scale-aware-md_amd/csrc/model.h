@@ -74,7 +74,7 @@ FitOffsets fit_offsets(const ModelHost& m);
 struct C4Host {
   double eps = 0, floor = 0, stride = 0;
   int n_int = 0, H = 0, act = 0, resnet = 0;
-  std::vector<float> table, film, ro, temb, mean, istd, w0t, b0, wh;
+  std::vector<float> table, film, ro, temb, mean, istd, wf, wb, b0, wh;
   float bh = 0.f;
   std::vector<double> bias;
 };
