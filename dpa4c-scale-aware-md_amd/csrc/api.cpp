@@ -102,10 +102,10 @@ struct dp_model {
   double* d_exp_pad = nullptr;
   double* d_nets = nullptr;
   // the fitting layers' weights of every type transposed ([out][in], at the
-  // layer's offset in the type's block of fit_t_stride): the input gradients'
-  // operand
+  // layer's offset in the type's block): the input gradients' operand. d_fit
+  // and d_fit_t hold one block of fit_stride elements per type.
   void* d_fit_t = nullptr;
-  size_t fit_t_stride = 0;
+  size_t fit_stride = 0;
   // mixed precision: per type and fitting layer, byte offsets into d_fitf of
   // the pre-split W (forward) and W^T (backward) fragments, -1 if absent
   void* d_fitf = nullptr;
@@ -436,7 +436,7 @@ void fit_types(dp_model* M, hipStream_t st, int nb, int Fmax, bool d_from_t, boo
   for (int t = 0; t < nt; ++t) {
     const int rows = M->type_off[t + 1] - M->type_off[t];
     active += rows > 0;
-    const int sp = rows > 0 ? fit_splits(rows, m.fit[0], Dn, M->ncu) : 1;
+    const int sp = rows > 0 ? fit_splits(rows, m.fit[0], Dn, M->ncu, f32) : 1;
     if (sp > 1) ws_need += (size_t)sp * rows * m.fit[0];
     const int ds = (fused_ddt && rows > 0) ? ddt_splits(rows, L3, M->ncu) : 1;
     if (ds > 1) ddt_need += (size_t)(ds + 1) * rows * 64;
@@ -478,11 +478,12 @@ void fit_types(dp_model* M, hipStream_t st, int nb, int Fmax, bool d_from_t, boo
       fst = M->fit_st[t];
       DPAMD_HIP(hipStreamWaitEvent(fst, M->fork_ev, 0));
     }
-    const E* P = static_cast<const E*>(M->d_fit) + (size_t)t * m.fit_block;
+    const E* P = static_cast<const E*>(M->d_fit) + (size_t)t * M->fit_stride;
     FitNet<E> net{};
     const int ins[3] = {Dn, m.fit[0], m.fit[1]};
     for (int k = 0; k < 3; ++k) {
       net.L[k].W = P + M->fo.W[k];
+      net.L[k].WT = static_cast<const E*>(M->d_fit_t) + (size_t)t * M->fit_stride + M->fo.W[k];
       net.L[k].b = P + M->fo.b[k];
       net.L[k].idt = M->fo.idt[k] >= 0 ? P + M->fo.idt[k] : nullptr;
       net.L[k].in = ins[k];
@@ -499,7 +500,7 @@ void fit_types(dp_model* M, hipStream_t st, int nb, int Fmax, bool d_from_t, boo
     const size_t r0 = (size_t)M->type_off[t];
     const size_t slab = (size_t)std::max(nb, 1) * Fmax;
     FitBufs<E> fb{};
-    fb.split = fit_splits(rows, m.fit[0], Dn, M->ncu);
+    fb.split = fit_splits(rows, m.fit[0], Dn, M->ncu, f32);
     if (fb.split > 1) fb.ws = split_ws + ws_off;
     ws_off += (size_t)fb.split * rows * m.fit[0];
     E* base = fitb;
@@ -513,7 +514,7 @@ void fit_types(dp_model* M, hipStream_t st, int nb, int Fmax, bool d_from_t, boo
       if constexpr (f32)
         ddt.W0T = static_cast<const char*>(M->d_fitf) + M->fitf_off[t][0][1];
       else
-        ddt.W0T = static_cast<const double*>(M->d_fit_t) + (size_t)t * M->fit_t_stride;
+        ddt.W0T = static_cast<const double*>(M->d_fit_t) + (size_t)t * M->fit_stride;
       ddt.items = items;
       ddt.pos0 = (int)r0;
       ddt.dT = dT;
@@ -713,8 +714,8 @@ void run_model_t(dp_model* M, hipStream_t st, int nloc, int nall, const int* d_n
     fa.slices = few_slices(L3);
     int tiles = 0;
     for (int t = 0; t < nt; ++t) {
-      const E* P = static_cast<const E*>(M->d_fit) + (size_t)t * m.fit_block;
-      const E* PT = static_cast<const E*>(M->d_fit_t) + (size_t)t * M->fit_t_stride;
+      const E* P = static_cast<const E*>(M->d_fit) + (size_t)t * M->fit_stride;
+      const E* PT = static_cast<const E*>(M->d_fit_t) + (size_t)t * M->fit_stride;
       FewNet<E>& net = fa.net[t];
       for (int k = 0; k < 3; ++k) {
         net.W[k] = P + M->fo.W[k];
@@ -1459,9 +1460,7 @@ int dp_create(const char* path, int gpu_rank, const void* file_content, size_t c
       // the nets are evaluated in fp32: round the parameters once here
       std::vector<float> emb32(emb.begin(), emb.end());
       pack_embedding_bf16(m, M->el, emb32);
-      const std::vector<float> fit32(m.fit_params.begin(), m.fit_params.end());
       upload(M->d_emb, emb32);
-      upload(M->d_fit, fit32);
       // fitting GEMM operands pre-split for the bf16 matrix cores: W0, W1,
       // W2 forward, W1 / W2 transposed, and W0 transposed tile-major for the
       // fused dE/dD -> dE/dT kernel (when it applies; otherwise dE/dD is
@@ -1483,18 +1482,24 @@ int dp_create(const char* path, int gpu_rank, const void* file_content, size_t c
       upload(M->d_fitf, frag);
     } else {
       upload(M->d_emb, emb);
-      upload(M->d_fit, m.fit_params);
     }
     M->fo = fit_offsets(m);
     {
       const int ins[3] = {m.emb[2] * m.axis, m.fit[0], m.fit[1]};
-      M->fit_t_stride = ((size_t)m.fit_block + 15) / 16 * 16;  // (16-byte aligned blocks)
+      M->fit_stride = ((size_t)m.fit_block + 15) / 16 * 16;  // (16-byte aligned blocks)
+      auto padded = [&](auto zero) {
+        std::vector<decltype(zero)> out(m.ntypes * M->fit_stride, zero);
+        for (int t = 0; t < m.ntypes; ++t)
+          std::copy_n(m.fit_params.begin() + (size_t)t * m.fit_block, m.fit_block,
+                      out.begin() + t * M->fit_stride);
+        return out;
+      };
       auto transposed = [&](auto zero) {
-        std::vector<decltype(zero)> out(m.ntypes * M->fit_t_stride, zero);
+        std::vector<decltype(zero)> out(m.ntypes * M->fit_stride, zero);
         for (int t = 0; t < m.ntypes; ++t)
           for (int k = 0; k < 3; ++k) {
             const double* W = m.fit_params.data() + (size_t)t * m.fit_block + M->fo.W[k];
-            auto* o = out.data() + t * M->fit_t_stride + M->fo.W[k];
+            auto* o = out.data() + t * M->fit_stride + M->fo.W[k];
             const int in = ins[k], on = m.fit[k];
             for (int i0 = 0; i0 < in; i0 += 32)
               for (int j0 = 0; j0 < on; j0 += 32)
@@ -1504,8 +1509,13 @@ int dp_create(const char* path, int gpu_rank, const void* file_content, size_t c
           }
         return out;
       };
-      if (mixed) upload(M->d_fit_t, transposed(0.0f));
-      else upload(M->d_fit_t, transposed(0.0));
+      if (mixed) {
+        upload(M->d_fit, padded(0.0f));
+        upload(M->d_fit_t, transposed(0.0f));
+      } else {
+        upload(M->d_fit, padded(0.0));
+        upload(M->d_fit_t, transposed(0.0));
+      }
     }
     M->bytes_peak = M->bytes_now;
     if (const char* g = std::getenv("DPAMD_GRAPH")) M->graph_on = std::atoi(g) != 0;

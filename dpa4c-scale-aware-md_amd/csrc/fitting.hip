@@ -215,8 +215,8 @@ __device__ __forceinline__ void gemm_store(const GemmArgs<T>& a, const typename 
   else gemm_store_rows<T, NT, EPI, false>(a, acc, row0, col0, zs, w, g, c);
 }
 
-// C = epi(A[MxK] B[KxN]); B(k,n) = TRANSB ? B[n*ldb + k] : B[k*ldb + n].
-// Block tile 64 x 16*NT: wave w owns rows 16w..16w+15 and all NT column tiles,
+// C = epi(A[MxK] B[KxN]); B(k,n) = TRANSB ? B[n*ldb + k] : B[k*ldb + n], for
+// fp32 operands that are not pre-split. Block tile 64 x 16*NT: wave w owns rows 16w..16w+15 and all NT column tiles,
 // so one A fragment feeds NT MFMAs. K advances 16 at a time through two LDS
 // buffers: the next chunk is fetched into registers while the current one is
 // multiplied, then stored into the other buffer (one barrier per chunk).
@@ -333,6 +333,140 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs<T> a) {
     __syncthreads();
   }
   gemm_store<T, NT, EPI>(a, acc, row0, col0, bid.z, w, g, c);
+}
+
+#define LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
+
+// The fp64 GEMM: C = epi(A[MxK] B[KxN]), B row-major. Nothing on the vector
+// unit runs beside an fp64 MFMA (measured: any vector instruction takes about
+// 4 cycles from the MFMA's 64), so the loop is built to hold few: block tile
+// 64 x 16 NT, wave w owning rows 16w .. 16w + 15 and all NT column tiles;
+// B chunks of 16 rows go straight into two LDS buffers (LDS DMA, uniform base +
+// a fixed 32-bit offset a lane), and A never passes through LDS: lane (g, c)
+// loads its own operands, rows c, k = 4 q + g.
+// AT: A is the descriptor D = T^T T[:, :16] of each row: K chunk a holds
+// D[row][16a + b] = sum_m T[m][a] T[m][b]; the lane keeps T[m][4 q + g] of its
+// row and loads T[0..3][a] a chunk (16 rows as one run, from the column-major
+// copy of T).
+// LDS rows are unpadded (the DMA writes linear runs); for even NT odd rows hold
+// neighbouring column tiles exchanged, so that two lane groups of a read fall
+// in different banks (odd NT: the row stride does it).
+// The first layer of 131,072 Cu atoms (N 240, K 1600, NT 5): 50 vector
+// instructions per 20 MFMAs and 2.37 ms with A and B staged through registers,
+// 26 and 2.17 ms now, MFMAs issued in 84 % of the cycles (the floor is
+// 1.42 ms at the 70.7 TFLOP/s of a large product). All 240 columns in one block
+// (NT 15: D formed once, 9 vector instructions per 20 MFMAs, but two waves per
+// SIMD instead of four) measured the same there and slower on few rows.
+template <int NT, bool AT, int EPI>
+__global__ __launch_bounds__(256, 2) void k_gemm_d(GemmArgs<double> a) {
+  constexpr int BK = 16, BN = 16 * NT, NI = BK * BN / 128, NJ = (NI + 3) / 4;
+  constexpr int G = NT % 5 == 0 ? 5 : NT % 4 == 0 ? 4 : NT % 3 == 0 ? 3 : 1;
+  __shared__ __align__(16) double Bs[2 * BK * BN];
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int3 bid = xcd_swizzle();
+  const int row0 = bid.y * 64, col0 = bid.x * BN;
+  // (rows past M repeat the last one and are not stored)
+  const int row = min(row0 + 16 * w + c, a.M - 1);
+  // the lane's granules (16 bytes) of a chunk: byte offset from its first row
+  unsigned offB[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    const int q = 64 * (w + 4 * j) + lane, kk = q / (BN / 2);
+    int col = 2 * (q % (BN / 2));
+    if (NT % 2 == 0) col ^= 16 * (kk & 1);
+    offB[j] = 8u * (unsigned)(kk * a.ldb + col);
+  }
+  auto issue = [&](int buf, int kc) {
+    const char* Bk = reinterpret_cast<const char*>(a.B + (long)kc * BK * a.ldb + col0);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+      if (w + 4 * j < NI)
+        __builtin_amdgcn_global_load_lds(reinterpret_cast<const double*>(Bk + offB[j]),
+                                         LDS_PTR(Bs + buf * BK * BN + 128 * (w + 4 * j)), 16, 0, 0);
+  };
+  double tb[4][4], ra[4];  // AT: T[m][4q + g]
+  unsigned offA;
+  if constexpr (AT) {
+    offA = 32u * (unsigned)row;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int m = 0; m < 4; ++m) tb[q][m] = a.Tt[(4 * q + g) * a.ldt + 4l * row + m];
+  } else {
+    offA = 8u * (unsigned)g;
+  }
+  const char* Arow = AT ? nullptr : reinterpret_cast<const char*>(a.A + (long)row * a.lda);
+  auto fetch = [&](int kc) {
+    if constexpr (AT) {
+      const char* Ta = reinterpret_cast<const char*>(a.Tt + kc * a.ldt);
+#pragma unroll
+      for (int m = 0; m < 4; ++m) ra[m] = *reinterpret_cast<const double*>(Ta + offA + 8 * m);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        ra[q] = *reinterpret_cast<const double*>(Arow + 8 * BK * kc + offA + 32 * q);
+    }
+  };
+  d4 acc[NT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n) acc[n] = d4{0.0, 0.0, 0.0, 0.0};
+  int kc0 = 0, nk = a.K / BK;
+  if (a.split > 1) {
+    const int per = (nk + a.split - 1) / a.split;
+    kc0 = bid.z * per;
+    nk = min(nk, kc0 + per);
+  }
+  // (a slice past the end of K keeps zeros: it is still stored, and summed)
+  if (kc0 < nk) {
+    issue(kc0 & 1, kc0);
+    fetch(kc0);
+  }
+  const int sw = NT % 2 == 0 ? 16 * (g & 1) : 0;
+  for (int kc = kc0; kc < nk; ++kc) {
+    const int buf = kc & 1;
+    double av[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if constexpr (AT)
+        av[q] = fma(ra[3], tb[q][3], fma(ra[2], tb[q][2], fma(ra[1], tb[q][1], ra[0] * tb[q][0])));
+      else
+        av[q] = ra[q];
+    }
+    // the chunk has landed (each wave waits for its own transfers, then the
+    // barrier), and no wave still reads the buffer the next one goes to
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (kc + 1 < nk) {
+      issue(buf ^ 1, kc + 1);
+      fetch(kc + 1);
+    }
+    const double* Be = Bs + buf * BK * BN + g * BN + c + sw;
+    const double* Bo = Bs + buf * BK * BN + g * BN + c - sw;
+    // B operands G tiles at a time, read a group ahead of their products (left
+    // to itself the compiler reads them two products ahead, less than the
+    // LDS latency)
+    double bf[2][G];
+    auto read = [&](int s) {
+#pragma unroll
+      for (int j = 0; j < G; ++j) {
+        const int q = s * G / NT, n = s * G % NT + j;
+        bf[s & 1][j] = (n % 2 ? Bo : Be)[4 * q * BN + 16 * n];
+      }
+    };
+    read(0);
+#pragma unroll
+    for (int s = 0; s < 4 * NT / G; ++s) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (s + 1 < 4 * NT / G) read(s + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < G; ++j) {
+        const int q = s * G / NT, n = s * G % NT + j;
+        acc[n] = mfma_f64(av[q], bf[s & 1][j], acc[n]);
+      }
+    }
+  }
+  gemm_store<double, NT, EPI>(a, acc, row0, col0, bid.z, w, g, c);
 }
 
 // fp32 GEMM on the bf16 matrix cores at fp32 accuracy (mixed precision):
@@ -483,16 +617,16 @@ __global__ __launch_bounds__(256) void k_splitk_tanh(int M, int N, int split,
 }
 
 // K slices for the first fitting layer: split only when the row blocks alone
-// leave the device short of work (fewer than four blocks per compute unit),
-// and keep at least 8 K chunks of 16 per slice (12,288-atom water: fitting
-// 0.717 -> 0.694 ms against a two-block target; an eight-block target with
-// 4-chunk slices was slower, 0.72 ms; the large types never split).
-int fit_splits(int rows, int N, int K, int ncu) {
+// leave the device short of work, and keep at least 8 K chunks of 16 per
+// slice. fp64: fewer than two blocks per compute unit (whole evaluation of
+// 12,288 water atoms 798 us, against 823 with a target of four; 24,000 atoms
+// 1,392 against 1,406; 3,993 and 98,304 atoms equal). fp32: fewer than four.
+int fit_splits(int rows, int N, int K, int ncu, bool f32) {
   const int cols = N % 128 == 0 ? N / 128 : N % 80 == 0 ? N / 80 : N % 64 == 0 ? N / 64 : N / 16;
   const long blocks = (long)cols * ((rows + 63) / 64);
   const int nk = K / 16;
   int split = 1;
-  while (blocks * split < 4L * ncu && nk / (2 * split) >= 8) split *= 2;
+  while (blocks * split < (f32 ? 4L : 2L) * ncu && nk / (2 * split) >= 8) split *= 2;
   return split;
 }
 
@@ -659,8 +793,6 @@ __global__ __launch_bounds__(kDtWaves * 64) void k_dT_any(int nb, int L3, int ax
 // of a row); dD (inspection only) is written when non-null.
 // Reference analog of the fused forward + gradient fitting entry:
 // deepmd-op/overlays/op/pt/graph_fitting.cu:728-757.
-#define LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
-
 struct DdtArgs {
   int rows, K, L3;
   const double* dZ;   // [rows][K]
@@ -1059,14 +1191,13 @@ static size_t ddt_lds_bytes(int K) {
 // transposed-B products plain or backward.
 template <class T, int NT, bool TRANSB, bool AT, int EPI>
 static void gemm_launch(hipStream_t st, const GemmArgs<T>& a, dim3 grid) {
-  if constexpr (sizeof(T) == 4) {
-    if (a.Bf) {  // B pre-split: the bf16 three-piece kernel (B's orientation is in the fragments)
-      hipLaunchKernelGGL((k_gemm3<NT, AT, EPI>), grid, dim3(256), 0, st, a);
-      DPAMD_LAUNCH_CHECK();
-      return;
-    }
+  if constexpr (sizeof(T) == 8) {
+    hipLaunchKernelGGL((k_gemm_d<NT, AT, EPI>), grid, dim3(256), 0, st, a);
+  } else if (a.Bf) {  // B pre-split: the bf16 three-piece kernel (B's orientation is in the fragments)
+    hipLaunchKernelGGL((k_gemm3<NT, AT, EPI>), grid, dim3(256), 0, st, a);
+  } else {
+    hipLaunchKernelGGL((k_gemm<T, NT, TRANSB, AT, EPI>), grid, dim3(256), 0, st, a);
   }
-  hipLaunchKernelGGL((k_gemm<T, NT, TRANSB, AT, EPI>), grid, dim3(256), 0, st, a);
   DPAMD_LAUNCH_CHECK();
 }
 
@@ -1085,16 +1216,21 @@ static void gemm_nt(hipStream_t st, const GemmArgs<T>& a) {
   throw HipError{hipErrorInvalidValue, "fitting GEMM: epilogue not available for this operand form"};
 }
 
-// Column tile (in MFMA tiles of 16 columns) of a fitting GEMM: the widest of
-// 8, 5, 4 or 1 that divides N; an fp64 GEMM over few rows takes 3 when it
-// divides N, for 5/3 as many blocks (a type of 8,192 rows, N = 240: 384 ->
-// 640 blocks of 64 rows; the layer is too short to fill the GPU otherwise).
-constexpr int kFewRows = 16384;
+// Column tile (in MFMA tiles of 16 columns) of a fitting GEMM.
+// fp32: the widest of 8, 5, 4 or 1 that divides N.
+// fp64: the widest of 8, 5, 4 or 3 that divides N and gives two blocks of 64
+// rows per compute unit (256); where none does, the narrowest that divides N,
+// for the most blocks (N 240: 3 up to 10,880 rows, then 5).
+constexpr int kFullGrid = 512;
 template <class T>
 static int col_tiles(int M, int N) {
   const int tiles = N / 16;
-  if (sizeof(T) == 8 && M < kFewRows && tiles % 3 == 0 && tiles % 8 != 0) return 3;
-  return tiles % 8 == 0 ? 8 : tiles % 5 == 0 ? 5 : tiles % 4 == 0 ? 4 : 1;
+  if (sizeof(T) == 4) return tiles % 8 == 0 ? 8 : tiles % 5 == 0 ? 5 : tiles % 4 == 0 ? 4 : 1;
+  const long rb = ((long)M + 63) / 64;
+  int nt = 1;
+  for (int k : {3, 4, 5, 8})
+    if (tiles % k == 0 && (nt == 1 || rb * (tiles / k) >= kFullGrid)) nt = k;
+  return nt;
 }
 template <bool TRANSB, class T>
 static void gemm(hipStream_t st, const GemmArgs<T>& a) {
@@ -1114,7 +1250,7 @@ static void gemm(hipStream_t st, const GemmArgs<T>& a) {
 }
 
 // First layer with A formed from T: the column tile is the widest of 8, 5, 4
-// or 1 MFMA tiles dividing N, as in gemm().
+// or 1 MFMA tiles dividing N (few rows split K instead, fit_splits).
 template <class T>
 static void gemm_at(hipStream_t st, const GemmArgs<T>& a) {
   if (a.M <= 0) return;
@@ -1123,6 +1259,14 @@ static void gemm_at(hipStream_t st, const GemmArgs<T>& a) {
   else if (tiles % 5 == 0) gemm_nt<T, 5, false, true>(st, a);
   else if (tiles % 4 == 0) gemm_nt<T, 4, false, true>(st, a);
   else gemm_nt<T, 1, false, true>(st, a);
+}
+
+// B of a product with a layer's transposed weights: fp64 the transposed copy
+// [out][in], fp32 the weights themselves (row stride ldw = out)
+template <class T>
+static void set_bt(GemmArgs<T>& g, const FitLayer<T>& L, int ldw) {
+  g.B = sizeof(T) == 8 ? L.WT : L.W;
+  g.ldb = sizeof(T) == 8 ? L.in : ldw;
 }
 
 template <class T>
@@ -1178,14 +1322,14 @@ void launch_fitting(hipStream_t st, const FitNet<T>& net, int rows, const T* D, 
   DPAMD_LAUNCH_CHECK();
   // backward: dH1 = [res2] Wo + dZ2 W2^T, dZ1 = dH1 idt1 (1 - T1^2)
   g = G{};
-  g.M = rows; g.N = F1; g.K = F2; g.A = b.dZa; g.lda = F2; g.B = net.L[2].W; g.ldb = F2;
+  g.M = rows; g.N = F1; g.K = F2; g.A = b.dZa; g.lda = F2; set_bt(g, net.L[2], F2);
   g.epi = 2; g.idt = net.L[1].idt; g.C = b.dZb; g.ldc = F1;
   g.dHin = net.L[2].idt ? net.Wo : nullptr; g.ld_dhin = 0; g.dH_out = b.dH; g.Tk = b.T1;
   g.Bf = net.L[2].WfT;
   gemm<true>(st, g);
   // dH0 = [res1] dH1 + dZ1 W1^T, dZ0 = dH0 (1 - H0^2)
   g = G{};
-  g.M = rows; g.N = F0; g.K = F1; g.A = b.dZb; g.lda = F1; g.B = net.L[1].W; g.ldb = F1;
+  g.M = rows; g.N = F0; g.K = F1; g.A = b.dZb; g.lda = F1; set_bt(g, net.L[1], F1);
   g.epi = 2; g.idt = nullptr; g.C = b.dZa; g.ldc = F0;
   g.dHin = net.L[1].idt ? b.dH : nullptr; g.ld_dhin = F1; g.dH_out = nullptr; g.Tk = b.H0;
   g.Bf = net.L[1].WfT;
@@ -1205,7 +1349,7 @@ void launch_fitting(hipStream_t st, const FitNet<T>& net, int rows, const T* D, 
   // fitting shapes the fused kernels do not cover (F0 != 240 or axis != 16):
   // the plain product dD = dZ0 W0^T, then launch_dT
   g = G{};
-  g.M = rows; g.N = Dn; g.K = F0; g.A = b.dZa; g.lda = F0; g.B = net.L[0].W; g.ldb = F0;
+  g.M = rows; g.N = Dn; g.K = F0; g.A = b.dZa; g.lda = F0; set_bt(g, net.L[0], F0);
   g.epi = 0; g.C = dD; g.ldc = Dn;
   gemm<true>(st, g);
 }

@@ -232,6 +232,7 @@ int embed_waves_bwd32(const EmbLayout&);
 template <class T>
 struct FitLayer {
   const T* W;    // [in][out]
+  const T* WT;   // [out][in]
   const T* b;    // [out]
   const T* idt;  // [out] or null
   int in, out;
@@ -257,7 +258,7 @@ struct FitBufs {
   T* ws;
 };
 // K slices fit_splits(rows, F0, Dn, compute units) for the first fitting layer
-int fit_splits(int rows, int N, int K, int ncu);
+int fit_splits(int rows, int N, int K, int ncu, bool f32);
 // The first layer reads its input either from D ([rows][L3*axis]) or, when
 // Tt is given (axis 16), forms D = T^T T[:, :16] on the fly from the
 // column-major copy of T (element (row, a, m) at Tt[a * ldt + 4 row + m]) and
