@@ -128,6 +128,22 @@ __device__ __forceinline__ double add_xor32(double v) {
   const unsigned l0 = l[0], l1 = l[1], h0 = h[0], h1 = h[1];
   return from32(h0, l0) + from32(h1, l1);
 }
+// Four values a lane summed over the four lane groups g of 16, group g keeping
+// the sum of value g: a transposing reduction (nine instructions, against
+// thirty for four full sums and a choice).
+__device__ __forceinline__ double sum_groups4(const double (&v)[4]) {
+  auto swap32 = [](double x, double y) {  // lanes < 32: x over the halves, others: y
+    const auto l = __builtin_amdgcn_permlane32_swap(lo32(x), lo32(y), true, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(hi32(x), hi32(y), true, false);
+    const unsigned l0 = l[0], l1 = l[1], h0 = h[0], h1 = h[1];
+    return from32(h0, l0) + from32(h1, l1);
+  };
+  const double a = swap32(v[0], v[2]), b = swap32(v[1], v[3]);
+  const auto l = __builtin_amdgcn_permlane16_swap(lo32(a), lo32(b), true, false);
+  const auto h = __builtin_amdgcn_permlane16_swap(hi32(a), hi32(b), true, false);
+  const unsigned l0 = l[0], l1 = l[1], h0 = h[0], h1 = h[1];
+  return from32(h0, l0) + from32(h1, l1);
+}
 __device__ __forceinline__ float add_xor16(float v) {
   const unsigned u = __builtin_bit_cast(unsigned, v);
   const auto s = __builtin_amdgcn_permlane16_swap(u, u, true, false);

@@ -791,6 +791,11 @@ __global__ __launch_bounds__(kDtWaves * 64) void k_dT_any(int nb, int L3, int ax
 // m) at Tt[a ldt + 4 pos + m]) with Tt pointing at the type's first row
 // (bucket position pos0); dT is in atom order (items[pos0 + row] is the atom
 // of a row); dD (inspection only) is written when non-null.
+// Vector instructions stop the fp64 MFMAs (k_gemm_d): per column group (60
+// MFMAs a wave) 144 of them, mostly the staging's and the flush's addresses and
+// the sums over the lane groups, took 2.44 ms for 131,072 Cu atoms; 64 with
+// uniform bases and one transposing sum, 2.30 ms, MFMAs issued in 80 % of the
+// cycles (98,304 water atoms, whole evaluation: 5.23 to 4.97 ms).
 // Reference analog of the fused forward + gradient fitting entry:
 // deepmd-op/overlays/op/pt/graph_fitting.cu:728-757.
 struct DdtArgs {
@@ -822,7 +827,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_dDdT(DdtArgs p) {
   // [WAVES][16 rows][4 m][16 columns], rows padded to kObRow doubles so that
   // the per-group writes (lane (g, c): row c, m = g) fall in distinct banks
   double* Ob = Ts + 2 * BM * 4;
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
   const int row0 = blockIdx.x * BM, wrow = row0 + 16 * w + c;  // this lane's row
   const bool rowok = wrow < p.rows;
   const int Dn = 16 * p.L3;
@@ -857,20 +862,29 @@ __global__ __launch_bounds__(WAVES * 64) void k_dDdT(DdtArgs p) {
   // columns 16a .. 16a + 15 (granule q: k = q / 8, columns 2 (q % 8) + 0, 1),
   // and T column a of the block's rows (granule q: row q / 2, m 2 (q % 2) + 0,
   // 1; rows past the type's end read its last row and are not used).
-  constexpr int NGB = K * 8, NGT = BM * 2;  // granules per group
+  // A transfer's address is a uniform base and a fixed 32-bit offset a lane.
+  constexpr int NB = K * 8 / 64, NT = BM * 2 / 64;  // wave transfers per group
+  constexpr int JB = (NB + WAVES - 1) / WAVES;
+  static_assert(NT <= WAVES, "one transfer of T a wave");
+  unsigned offB[JB];
+#pragma unroll
+  for (int u = 0; u < JB; ++u) {
+    const int q = 64 * (w + WAVES * u) + lane;
+    offB[u] = 8u * (unsigned)((q >> 3) * Dn + 2 * (q & 7));
+  }
+  const int qt = 64 * w + lane;
+  const unsigned offT = 32u * (unsigned)min(row0 + (qt >> 1), p.rows - 1) + 16u * (qt & 1);
   auto issue = [&](int buf, int a) {
-    for (int i = w; 64 * i < NGB; i += WAVES) {
-      const int q = 64 * i + lane;
-      if (q < NGB)
-        __builtin_amdgcn_global_load_lds(p.W0T + (long)(q >> 3) * Dn + 16 * a + 2 * (q & 7),
-                                         LDS_PTR(Bs + buf * K * 16 + 128 * i), 16, 0, 0);
-    }
-    for (int i = w; 64 * i < NGT; i += WAVES) {
-      const int q = 64 * i + lane;
-      const int r = min(row0 + (q >> 1), p.rows - 1);
-      __builtin_amdgcn_global_load_lds(p.Tt + (long)a * p.ldt + 4L * r + 2 * (q & 1),
-                                       LDS_PTR(Ts + buf * BM * 4 + 128 * i), 16, 0, 0);
-    }
+    const char* W0 = reinterpret_cast<const char*>(p.W0T + 16 * a);
+    const char* T0 = reinterpret_cast<const char*>(p.Tt + (long)a * p.ldt);
+#pragma unroll
+    for (int u = 0; u < JB; ++u)
+      if (w + WAVES * u < NB)
+        __builtin_amdgcn_global_load_lds(reinterpret_cast<const double*>(W0 + offB[u]),
+                                         LDS_PTR(Bs + buf * K * 16 + 128 * (w + WAVES * u)), 16, 0, 0);
+    if (w < NT)
+      __builtin_amdgcn_global_load_lds(reinterpret_cast<const double*>(T0 + offT),
+                                       LDS_PTR(Ts + buf * BM * 4 + 128 * w), 16, 0, 0);
   };
   auto col_of = [&](int i) { return i + 16 < p.L3 ? i + 16 : i + 16 - p.L3; };
 
@@ -879,7 +893,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_dDdT(DdtArgs p) {
     const int a = col_of(i), buf = (i - i0) & 1;
     // group i has landed (each wave waits for its own transfers, then the
     // barrier), and no wave still reads the buffer group i + 1 goes to
-    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if (i + 1 < i1) issue(buf ^ 1, col_of(i + 1));
     // D'[b][row] over K: register r of lane (g, c) = dD[row c][a][g + 4r]
     // two independent accumulation chains (the halves of K), operands read
@@ -913,10 +927,9 @@ __global__ __launch_bounds__(WAVES * 64) void k_dDdT(DdtArgs p) {
       v = fma(acc[1], Tc[1][m], v);
       v = fma(acc[2], Tc[2][m], v);
       v = fma(acc[3], Tc[3][m], v);
-      v = add_xor32(add_xor16(v));
       s[m] = v;
     }
-    Obw[c * kObRow + g * 16 + (a & 15)] = g == 0 ? s[0] : g == 1 ? s[1] : g == 2 ? s[2] : s[3];
+    Obw[c * kObRow + g * 16 + (a & 15)] = sum_groups4(s);
     // second term: T[row][m][a]
     const double* tr = Ts + buf * BM * 4 + (16 * w + c) * 4;
 #pragma unroll
@@ -933,13 +946,16 @@ __global__ __launch_bounds__(WAVES * 64) void k_dDdT(DdtArgs p) {
     if (a >= 16 && ((a & 15) == 15 || a == p.L3 - 1)) {
       wave_lds_sync();
       const int abase = a & ~15, na = a - abase + 1;
+      // pass rl: row rl of the wave, lane = (m, al); the row's address is
+      // uniform
+      const int al = lane & 15, off = (lane >> 4) * p.L3 + al;
+      const int left = p.rows - row0 - 16 * w;  // rows of this wave
 #pragma unroll
       for (int rl = 0; rl < 16; ++rl) {
-        // pass rl: row rl of the wave, lane = (m, al)
-        const int atom = __shfl(my_atom, rl, 64);
-        const int m = lane >> 4, al = lane & 15;
-        if (al < na && row0 + 16 * w + rl < p.rows)
-          p.dT[((long)atom * 4 + m) * p.L3 + abase + al] = Obw[kObRow * rl + lane];
+        const int atom = __builtin_amdgcn_readlane(my_atom, rl);
+        double* out = p.dT + (long)atom * 4 * p.L3 + abase;
+        const double v = Obw[kObRow * rl + lane];
+        if (rl < left && al < na) out[off] = v;
       }
       wave_lds_sync();
     }
