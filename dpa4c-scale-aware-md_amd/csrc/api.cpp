@@ -969,28 +969,30 @@ int build_standalone_nlist(dp_model* M, hipStream_t st, int nloc, const double* 
   int* cstart = need<int>(M, M->cell_start, (size_t)ncell + 1);
   int* crank = need<int>(M, M->cell_rank, (size_t)nall);
   CellAtom* sorted = need<CellAtom>(M, M->sorted, (size_t)nall);
-  // the wrap also clears the cell counts (and gives nall when there are no
-  // ghosts); the ghost placement gives nall otherwise
-  launch_wrap(st, nloc, d_coord, d_atype, bp, ext, ext_type, mapping, sfrac, ncell + 1, ccount,
-              nf > 0 ? nullptr : nall_d);
+  // the first kernel also wraps the atoms and clears the cell counts; the last
+  // of the ghosts' also gives nall and assigns the cells
   if (nf > 0) {
     const long nc = (long)bp.nshift * ghost_tiles(nloc);  // per (shift, tile of atoms)
     int* count = need<int>(M, M->flags, (size_t)nc);
     int* first = need<int>(M, M->gpos, (size_t)nc);
-    launch_ghost_count(st, nloc, bp, sfrac, count);
+    launch_ghost_count(st, nloc, d_coord, d_atype, bp, ext, ext_type, mapping, sfrac, ncell + 1,
+                       ccount, count);
     const size_t tb = scan_temp_bytes((int)nc);
     void* tmp = need<char>(M, M->scan_tmp, tb);
-    exclusive_scan_int(st, count, first, (int)nc, tmp, tb);
-    launch_ghost_place(st, nloc, bp, sfrac, count, first, ext, ext_type, mapping, nall_d);
+    const bool scan = ghost_scan_needed(nc);
+    if (scan) exclusive_scan_int(st, count, first, (int)nc, tmp, tb);
+    launch_ghost_place(st, nloc, bp, sfrac, count, scan ? first : nullptr, ext, ext_type, mapping,
+                       nall_d, cell_of, crank, ccount);
+  } else {
+    launch_wrap(st, nloc, d_coord, d_atype, bp, ext, ext_type, mapping, ncell + 1, ccount, nall_d);
+    launch_cell_assign(st, nloc, bp, ext, cell_of, crank, ccount);
   }
-  // cells
-  launch_cell_assign(st, nall, nall_d, bp, ext, cell_of, crank, ccount);
   {
     const size_t tb = scan_temp_bytes(ncell + 1);
     void* tmp = need<char>(M, M->scan_tmp, tb);
-    exclusive_scan_int(st, ccount, cstart, ncell + 1, tmp, tb);
+    if (cell_scan_needed(ncell)) exclusive_scan_int(st, ccount, cstart, ncell + 1, tmp, tb);
   }
-  launch_cell_scatter(st, nall, nall_d, cell_of, crank, cstart, ext, ext_type, sorted);
+  launch_cell_scatter(st, nall, nall_d, ncell, ccount, cell_of, crank, cstart, ext, ext_type, sorted);
   if (np.unsorted) launch_cell_order(st, ncell, cstart, sorted);
   record(M, st, kStGeom + 1);
   int* nlist = need<int>(M, M->nlist, (size_t)std::max(nloc, 1) * m.nnei);

@@ -157,26 +157,32 @@ struct DescArgs {
 // Neighbour stage
 // also clears clear[0 .. nclear) and, when nall is given, sets *nall = nloc
 void launch_wrap(hipStream_t, int nloc, const double* coord, const int* atype, const BoxParams&,
-                 double* ext, int* ext_type, int* mapping, double* sfrac, int nclear, int* clear,
-                 int* nall);
-// Ghost images in (shift, atom) order: per shift, the number of images of each
+                 double* ext, int* ext_type, int* mapping, int nclear, int* clear, int* nall);
+// Ghost images in (shift, atom) order: wraps the atoms (ext, ext_type, mapping,
+// sfrac), clears clear[0 .. nclear) and counts, per shift, the images of each
 // tile of atoms that land in the extended region (count[s * ghost_tiles(nloc)
-// + tile]); then, from the exclusive scan of those counts, the images
-// themselves (coordinates, types and mapping after the nloc local atoms).
+// + tile]); then places them by the counts' exclusive scan `first`, which may
+// be null where ghost_scan_needed(number of counts) is false, also giving
+// *nall = nloc + the number of ghosts and every atom's cell and its rank there.
 int ghost_tiles(int nloc);
-void launch_ghost_count(hipStream_t, int nloc, const BoxParams&, const double* sfrac, int* count);
-// (also *nall = nloc + the number of ghosts)
+void launch_ghost_count(hipStream_t, int nloc, const double* coord, const int* atype,
+                        const BoxParams&, double* ext, int* ext_type, int* mapping, double* sfrac,
+                        int nclear, int* clear, int* count);
+bool ghost_scan_needed(long counts);
 void launch_ghost_place(hipStream_t, int nloc, const BoxParams&, const double* sfrac,
                         const int* count, const int* first, double* ext, int* ext_type,
-                        int* mapping, int* nall);
-// Cell kernels over cap atoms, or over *d_count of them when d_count is given
-// (a count produced on the device, at most cap).
-// (cell_rank: an atom's rank within its cell, from the count)
-void launch_cell_assign(hipStream_t, int cap, const int* d_count, const BoxParams&,
-                        const double* ext, int* cell_of, int* cell_rank, int* cell_count);
-void launch_cell_scatter(hipStream_t, int cap, const int* d_count, const int* cell_of,
-                         const int* cell_rank, const int* cell_start, const double* ext,
-                         const int* ext_type, CellAtom* sorted);
+                        int* mapping, int* nall, int* cell_of, int* cell_rank, int* cell_count);
+// Cells of a box without ghost images.
+void launch_cell_assign(hipStream_t, int nloc, const BoxParams&, const double* ext, int* cell_of,
+                        int* cell_rank, int* cell_count);
+// Cell-sorted records of cap atoms, or of *d_count when given (a count produced
+// on the device, at most cap). cell_start is the exclusive scan of the ncell + 1
+// counts where cell_scan_needed(ncell), and written otherwise.
+bool cell_scan_needed(int ncell);
+void launch_cell_scatter(hipStream_t, int cap, const int* d_count, int ncell,
+                         const int* cell_count, const int* cell_of, const int* cell_rank,
+                         int* cell_start, const double* ext, const int* ext_type,
+                         CellAtom* sorted);
 // atoms of each cell in ascending index order (reproducible candidate order)
 void launch_cell_order(hipStream_t, int ncell, const int* cell_start, CellAtom* sorted);
 // p[0 .. n) = v (a kernel rather than a memset node, so it can be captured)
