@@ -1,5 +1,7 @@
 // Fused environment matrix + embedding net + descriptor contraction on
-// gfx950 FP64 MFMA (v_mfma_f64_16x16x4f64), and its backward.
+// gfx950 FP64 MFMA (v_mfma_f64_16x16x4f64), and its backward, slot by slot: for
+// models with a net that has no short enough expansion (expand.hip serves the
+// others).
 //
 // Work unit: one wave owns one (centre i, neighbour section tj) item and walks
 // its real slots in tiles of 16; a workgroup holds the padded weights of one

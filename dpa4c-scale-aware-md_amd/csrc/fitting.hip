@@ -474,72 +474,71 @@ __global__ __launch_bounds__(256, 2) void k_gemm_d(GemmArgs<double> a) {
 // a.Bf [ceil(K/32)][N/16][3][64 lanes] (8 bf16 each: lane 16g + c of (chunk
 // h, column tile n) holds the pieces of B(32h + 8g + e, 16n + c), e = 0..7,
 // zero past K). Block tile 64 x 16 NT, wave w rows 16w..16w+15 as in k_gemm;
-// K advances 32 at a time: the A chunk (fp32) and the block's B fragments
-// (NT tiles) go through two LDS buffers, each wave splits its A fragment
-// (row 16w + c, k 8g..8g+7) once per chunk and runs six bf16 MFMAs per column
-// tile (mfma3). On gfx950 the fp32 16x16x4 MFMA is barely faster than the
-// VALU; the bf16 form with the six-product split does about twice its work
-// per unit time. AT: A is D = T^T T[:, :16] formed while staging; chunk kc
-// holds D columns 32kc.. 32kc + 31 (a = 2kc, 2kc + 1), thread (row, part)
-// stages columns 8 part .. 8 part + 7 and keeps T[m][8 (part % 2) + e].
+// K advances 32 at a time. As in k_gemm_d the B fragments (NT tiles) go
+// straight into two LDS buffers and A never passes through LDS: lane (g, c)
+// loads k 8g .. 8g + 7 of row 16w + c, splits them once per chunk and runs six
+// bf16 MFMAs per column tile (mfma3). On gfx950 the fp32 16x16x4 MFMA is barely
+// faster than the VALU; the bf16 form with the six-product split does about
+// twice its work per unit time. AT: A is D = T^T T[:, :16]; chunk kc holds D
+// columns 32kc .. 32kc + 31 (a = 2kc, 2kc + 1), the lane keeps T[m][b], b = 8 (g
+// % 2) + e, and loads T[0..3][2kc + g / 2] a chunk. With both
+// operands staged through registers and A through LDS, whole evaluations took
+// 5,283 us at 128,000 HEA atoms, 671 at 6,750 and 643 at 16,384 Cu atoms; now
+// 4,995, 618 and 589, with the same bits.
 template <int NT, bool AT, int EPI>
 __global__ __launch_bounds__(256) void k_gemm3(GemmArgs<float> a) {
-  constexpr int BM = 64, BK = 32, BN = 16 * NT, ALD = BK + 4;
-  __shared__ __align__(16) float As[2][BM * ALD];
-  __shared__ __align__(16) bf8 Bs[2][NT * 3 * 64];
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, g = lane >> 4, c = lane & 15;
+  constexpr int BM = 64, BK = 32, BN = 16 * NT;
+  constexpr int NI = NT * 3, NJ = (NI + 3) / 4;  // wave transfers of a chunk's B, per wave
+  __shared__ __align__(16) bf8 Bs[2 * NT * 192];
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int3 bid = xcd_swizzle();
   const int row0 = bid.y * BM, col0 = bid.x * BN;
   const int ntile = a.N / 16, tile0 = col0 / 16;
-  const bf8* Bf = static_cast<const bf8*>(a.Bf);
-  // staging share: row sr, k columns sk .. sk + 7 of the chunk
-  const int sr = tid >> 2, part = tid & 3, sk = 8 * part;
-  const int grow = row0 + sr;
-  const float* arow = grow < a.M ? (AT ? a.Tt + 4 * (long)grow : a.A + (long)grow * a.lda) : nullptr;
-  float tb[4][8];
-  if constexpr (AT) {
+  // (rows past M repeat the last one and are not stored)
+  const int row = min(row0 + 16 * w + c, a.M - 1);
+  auto issue = [&](int buf, int kc) {
+    const bf8* src = static_cast<const bf8*>(a.Bf) + ((long)kc * ntile + tile0) * 192;
 #pragma unroll
-    for (int m = 0; m < 4; ++m)
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        tb[m][e] = arow ? arow[(8 * (part & 1) + e) * a.ldt + m] : 0.0f;
-  }
-  float ra[8];
-  bf8 rb[(NT * 3 * 64 + 255) / 256];
-  auto fetch = [&](int kc) {
-    if constexpr (AT) {
-      // ra[m] = T[m][a] of this row, a = 2 kc + part / 2
-      const int ac = 2 * kc + (part >> 1);
-#pragma unroll
-      for (int m = 0; m < 4; ++m) ra[m] = arow ? arow[(long)ac * a.ldt + m] : 0.0f;
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int k = 32 * kc + sk + e;
-        ra[e] = (arow && k < a.K) ? arow[k] : 0.0f;
-      }
-    }
-    const bf8* src = Bf + ((long)kc * ntile + tile0) * 192;
-#pragma unroll
-    for (int u = 0; u < (NT * 192 + 255) / 256; ++u) {
-      const int q = tid + 256 * u;
-      if (q < NT * 192) rb[u] = src[q];
+    for (int j = 0; j < NJ; ++j) {
+      const int i = w + 4 * j;
+      if (i < NI)
+        __builtin_amdgcn_global_load_lds(src + 64 * i + lane, LDS_PTR(Bs + buf * NT * 192 + 64 * i),
+                                         16, 0, 0);
     }
   };
-  auto stash = [&](int buf) {
-    float* dst = As[buf] + sr * ALD + sk;
-    if constexpr (AT) {
+  float tb[4][8], v[8];
+  f4 ra[2];
+  if constexpr (AT) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e)
-        dst[e] = ra[0] * tb[0][e] + ra[1] * tb[1][e] + ra[2] * tb[2][e] + ra[3] * tb[3][e];
-    } else {
+    for (int e = 0; e < 8; ++e) {
+      const f4 t = *reinterpret_cast<const f4*>(a.Tt + (8 * (g & 1) + e) * a.ldt + 4L * row);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) dst[e] = ra[e];
+      for (int m = 0; m < 4; ++m) tb[m][e] = t[m];
     }
+  }
+  const unsigned hi = AT ? 4u * (unsigned)a.ldt * (g >> 1) : 0u;  // bytes to column a = 2 kc + g / 2
+  const char* Arow = AT ? nullptr : reinterpret_cast<const char*>(a.A + (long)row * a.lda);
+  auto fetch = [&](int kc) {
+    if constexpr (AT) {
+      // (an odd number of columns: B holds zeros past K, any column will do)
+      const unsigned off = 16u * (unsigned)row + (16 * (2 * kc + 1) < a.K ? hi : 0u);
+      ra[0] = *reinterpret_cast<const f4*>(
+          reinterpret_cast<const char*>(a.Tt + 2L * kc * a.ldt) + off);
+    } else {
+      // (past K, where B holds zeros, the row's last eight values)
+      const char* src = Arow + 4 * min(BK * kc + 8 * g, a.K - 8);
+      ra[0] = *reinterpret_cast<const f4*>(src);
+      ra[1] = *reinterpret_cast<const f4*>(src + 16);
+    }
+  };
+  auto operand = [&]() {
 #pragma unroll
-    for (int u = 0; u < (NT * 192 + 255) / 256; ++u) {
-      const int q = tid + 256 * u;
-      if (q < NT * 192) Bs[buf][q] = rb[u];
+    for (int e = 0; e < 8; ++e) {
+      if constexpr (AT)
+        v[e] = ra[0][0] * tb[0][e] + ra[0][1] * tb[1][e] + ra[0][2] * tb[2][e] + ra[0][3] * tb[3][e];
+      else
+        v[e] = ra[e / 4][e % 4];
     }
   };
   f4 acc[NT];
@@ -552,22 +551,28 @@ __global__ __launch_bounds__(256) void k_gemm3(GemmArgs<float> a) {
     nk = min(nk, kc0 + per);
   }
   if (kc0 < nk) {
+    issue(kc0 & 1, kc0);
     fetch(kc0);
-    stash(kc0 & 1);
   }
-  __syncthreads();
   for (int kc = kc0; kc < nk; ++kc) {
     const int buf = kc & 1;
-    if (kc + 1 < nk) fetch(kc + 1);
-    const Split3 xa = split3(As[buf] + (16 * w + c) * ALD + 8 * g);
+    operand();
+    // the chunk has landed (each wave waits for its own transfers, then the
+    // barrier), and no wave still reads the buffer the next one goes to
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (kc + 1 < nk) {
+      issue(buf ^ 1, kc + 1);
+      fetch(kc + 1);
+    }
     // each column tile's B pieces are read from LDS one tile ahead of its
     // products (scheduling barriers keep the compiler from sinking the reads
     // to their use)
     auto bp = [&](int n) {
-      const bf8* b = Bs[buf] + n * 192 + lane;
+      const bf8* b = Bs + buf * NT * 192 + n * 192 + lane;
       return Split3{b[0], b[64], b[128]};
     };
     Split3 bc = bp(0);
+    const Split3 xa = split3(v);
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
       Split3 bn = bc;
@@ -577,8 +582,6 @@ __global__ __launch_bounds__(256) void k_gemm3(GemmArgs<float> a) {
       __builtin_amdgcn_sched_barrier(0);
       bc = bn;
     }
-    if (kc + 1 < nk) stash(buf ^ 1);
-    __syncthreads();
   }
   gemm_store<float, NT, EPI>(a, acc, row0, col0, bid.z, w, g, c);
 }
