@@ -215,39 +215,23 @@ __device__ __forceinline__ void gemm_store(const GemmArgs<T>& a, const typename 
   else gemm_store_rows<T, NT, EPI, false>(a, acc, row0, col0, zs, w, g, c);
 }
 
-// C = epi(A[MxK] B[KxN]); B(k,n) = TRANSB ? B[n*ldb + k] : B[k*ldb + n], for
-// fp32 operands that are not pre-split. Block tile 64 x 16*NT: wave w owns rows 16w..16w+15 and all NT column tiles,
-// so one A fragment feeds NT MFMAs. K advances 16 at a time through two LDS
-// buffers: the next chunk is fetched into registers while the current one is
-// multiplied, then stored into the other buffer (one barrier per chunk).
-// AT: A is the descriptor D = T^T T[:, :16] of each row, formed while staging:
-// K chunk a holds D[row][16a + b] = sum_m T[m][a] T[m][b]; thread (r, part)
-// keeps T[m][4 part .. 4 part + 3] of row r in registers and fetches the 4
-// values T[0..3][a] per chunk (contiguous in the column-major copy of T, so a
-// wave reads 16 rows as one run) instead of 16 values of D.
-template <class T, int NT, bool TRANSB, bool AT, int EPI>
-__global__ __launch_bounds__(256) void k_gemm(GemmArgs<T> a) {
+// fp32 C = A[MxK] B[KxN] with B(k, n) = B[n ldb + k], on the fp32 MFMA: the input
+// gradient dE/dD of fitting shapes whose transposed first layer is not pre-split
+// (every other fp32 product has its bf16 fragments). Block tile 64 x 16 NT: wave
+// w owns rows 16w..16w+15 and all NT column tiles, so one A fragment feeds NT
+// MFMAs. K advances 16 at a time through two LDS buffers: the next chunk is
+// fetched into registers while the current one is multiplied, then stored into
+// the other buffer (one barrier per chunk).
+template <int NT>
+__global__ __launch_bounds__(256) void k_gemm(GemmArgs<float> a) {
   constexpr int BM = 64, BK = 16, BN = 16 * NT;
   constexpr int ALD = BK + 1, BLD = BN + 1;
   constexpr int NA = BM * BK / 256, NB = (BK * BN + 255) / 256;
-  static_assert(!AT || NA == 4, "AT staging assumes 4 A elements per thread");
-  __shared__ T As[2][BM * ALD];
-  __shared__ T Bs[2][BK * BLD];
+  __shared__ float As[2][BM * ALD];
+  __shared__ float Bs[2][BK * BLD];
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, g = lane >> 4, c = lane & 15;
   const int3 bid = xcd_swizzle();
   const int row0 = bid.y * BM, col0 = bid.x * BN;
-  // AT: this thread's row and column quarter, and T[m][4 part + j] of the row
-  const int at_r = tid >> 2, at_part = tid & 3;
-  const T* at_row = nullptr;  // T[.][0][row] of this thread's row
-  T tb[4][4];
-  if constexpr (AT) {
-    if (row0 + at_r < a.M) at_row = a.Tt + 4 * (long)(row0 + at_r);
-#pragma unroll
-    for (int m = 0; m < 4; ++m)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        tb[m][j] = at_row ? at_row[(4 * at_part + j) * a.ldt + m] : T(0);
-  }
   // element offsets of this thread's share of a K chunk, fixed over chunks
   int offA[NA], ldsA[NA], offB[NB], ldsB[NB];
 #pragma unroll
@@ -258,81 +242,46 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs<T> a) {
   }
 #pragma unroll
   for (int u = 0; u < NB; ++u) {
-    const int q = tid + 256 * u;
-    if (q < BK * BN) {
-      if (!TRANSB) {
-        const int kk = q / BN, n = q % BN;
-        offB[u] = kk * a.ldb + col0 + n;
-        ldsB[u] = kk * BLD + n;
-      } else {
-        const int n = q / BK, kk = q % BK;
-        offB[u] = (col0 + n) * a.ldb + kk;
-        ldsB[u] = kk * BLD + n;
-      }
-    } else {
-      offB[u] = -1;
-      ldsB[u] = 0;
-    }
+    const int q = tid + 256 * u, n = q / BK, kk = q % BK;
+    offB[u] = q < BK * BN ? (col0 + n) * a.ldb + kk : -1;
+    ldsB[u] = kk * BLD + n;
   }
-  T ra[NA], rb[NB];
+  float ra[NA], rb[NB];
   auto fetch = [&](int k0) {
-    const T* Bk = TRANSB ? a.B + k0 : a.B + (long)k0 * a.ldb;
-    if constexpr (AT) {
-      // ra[m] = T[m][a] of this thread's row, a = k0 / 16
 #pragma unroll
-      for (int m = 0; m < 4; ++m) ra[m] = at_row ? at_row[(k0 >> 4) * a.ldt + m] : T(0);
-    } else {
-      const T* Ak = a.A + k0;
+    for (int u = 0; u < NA; ++u) ra[u] = offA[u] >= 0 ? a.A[k0 + offA[u]] : 0.0f;
 #pragma unroll
-      for (int u = 0; u < NA; ++u) ra[u] = offA[u] >= 0 ? Ak[offA[u]] : T(0);
-    }
-#pragma unroll
-    for (int u = 0; u < NB; ++u) rb[u] = offB[u] >= 0 ? Bk[offB[u]] : T(0);
+    for (int u = 0; u < NB; ++u) rb[u] = offB[u] >= 0 ? a.B[k0 + offB[u]] : 0.0f;
   };
   auto stash = [&](int buf) {
-    if constexpr (AT) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        As[buf][at_r * ALD + 4 * at_part + j] =
-            ra[0] * tb[0][j] + ra[1] * tb[1][j] + ra[2] * tb[2][j] + ra[3] * tb[3][j];
-    } else {
-#pragma unroll
-      for (int u = 0; u < NA; ++u) As[buf][ldsA[u]] = ra[u];
-    }
+    for (int u = 0; u < NA; ++u) As[buf][ldsA[u]] = ra[u];
 #pragma unroll
     for (int u = 0; u < NB; ++u)
       if (offB[u] >= 0) Bs[buf][ldsB[u]] = rb[u];
   };
-  typename Frag<T>::V acc[NT];
+  f4 acc[NT];
 #pragma unroll
-  for (int n = 0; n < NT; ++n) acc[n] = typename Frag<T>::V{0, 0, 0, 0};
-  int kc0 = 0, nk = a.K / BK;
-  if (a.split > 1) {
-    const int per = (nk + a.split - 1) / a.split;
-    kc0 = bid.z * per;
-    nk = min(nk, kc0 + per);
-  }
-  // (a slice past the end of K keeps zeros: it is still stored, and summed)
-  if (kc0 < nk) {
-    fetch(kc0 * BK);
-    stash(kc0 & 1);
-  }
+  for (int n = 0; n < NT; ++n) acc[n] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+  const int nk = a.K / BK;
+  fetch(0);
+  stash(0);
   __syncthreads();
-  for (int kc = kc0; kc < nk; ++kc) {
+  for (int kc = 0; kc < nk; ++kc) {
     const int buf = kc & 1;
     if (kc + 1 < nk) fetch((kc + 1) * BK);
-    const T* Ab = As[buf] + (16 * w + c) * ALD;
-    const T* Bb = Bs[buf];
+    const float* Ab = As[buf] + (16 * w + c) * ALD;
+    const float* Bb = Bs[buf];
 #pragma unroll
     for (int q = 0; q < BK / 4; ++q) {
-      const T av = Ab[4 * q + g];
+      const float av = Ab[4 * q + g];
 #pragma unroll
       for (int n = 0; n < NT; ++n) acc[n] = mfma(av, Bb[(4 * q + g) * BLD + 16 * n + c], acc[n]);
     }
     if (kc + 1 < nk) stash(buf ^ 1);
     __syncthreads();
   }
-  gemm_store<T, NT, EPI>(a, acc, row0, col0, bid.z, w, g, c);
+  gemm_store<float, NT, 0>(a, acc, row0, col0, 0, w, g, c);
 }
 
 #define LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
@@ -1214,8 +1163,10 @@ static void gemm_launch(hipStream_t st, const GemmArgs<T>& a, dim3 grid) {
     hipLaunchKernelGGL((k_gemm_d<NT, AT, EPI>), grid, dim3(256), 0, st, a);
   } else if (a.Bf) {  // B pre-split: the bf16 three-piece kernel (B's orientation is in the fragments)
     hipLaunchKernelGGL((k_gemm3<NT, AT, EPI>), grid, dim3(256), 0, st, a);
+  } else if constexpr (TRANSB && EPI == 0) {
+    hipLaunchKernelGGL(k_gemm<NT>, grid, dim3(256), 0, st, a);
   } else {
-    hipLaunchKernelGGL((k_gemm<T, NT, TRANSB, AT, EPI>), grid, dim3(256), 0, st, a);
+    throw HipError{hipErrorInvalidValue, "fitting GEMM: no bf16 fragments of this layer"};
   }
   DPAMD_LAUNCH_CHECK();
 }
