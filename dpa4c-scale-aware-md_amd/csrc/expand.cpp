@@ -125,10 +125,7 @@ void coefficients(const ModelHost& m, const std::vector<int>& pairs, int n,
     ld tail = 0.0L;
     for (int k = n - 1; k >= 16; --k) {
       ld a = 0.0L;
-      for (int f = 0; f < F; ++f) {
-        const ld v = std::fabs(coef[p][(size_t)k * F + f]);
-        a = v <= a ? a : v;  // (a NaN is kept)
-      }
+      for (int f = 0; f < F; ++f) a = std::max(a, std::fabs(coef[p][(size_t)k * F + f]));
       tail += a;
       if (!(tail < gmax * 0x1p-55L)) break;
       if (k % 16 == 0 && k <= std::min(n - 16, kExpandMaxTerms)) terms[p] = k;
@@ -140,6 +137,10 @@ void coefficients(const ModelHost& m, const std::vector<int>& pairs, int n,
 
 bool build_expansion(const ModelHost& m, ExpandHost& e) {
   const int np = m.ntypes * m.ntypes, F = m.emb[2];
+  // (finite parameters give finite coefficients: every layer is a tanh)
+  for (const auto* v : {&m.emb_params, &m.davg, &m.dstd})
+    for (double x : *v)
+      if (!std::isfinite(x)) return false;
   std::vector<std::vector<ld>> coef(np);
   std::vector<int> terms(np, 0);
   for (const int n : {112, 176, 304}) {

@@ -19,6 +19,12 @@ bool emb_supported(int, int, int) { return true; }
 }  // namespace dpamd
 using ld = long double;
 
+// the larger magnitude, NaN if either is
+static double larger(double a, ld b) {
+  const double v = std::fabs((double)b);
+  return v <= a || std::isnan(a) ? a : v;
+}
+
 int main(int argc, char** argv) {
   for (int q = 1; q < argc; ++q) {
     std::ifstream in(argv[q], std::ios::binary);
@@ -102,9 +108,9 @@ int main(int argc, char** argv) {
             g += C[(size_t)k * F + f] * T[k];
             d += C[(size_t)k * F + f] * D[k];
           }
-          eg = std::fmax(eg, std::fabs((double)(g - h[f])));
-          ed = std::fmax(ed, std::fabs((double)(d * dxds - t[f])));
-          gm = std::fmax(gm, std::fabs((double)h[f]));
+          eg = larger(eg, g - h[f]);
+          ed = larger(ed, d * dxds - t[f]);
+          gm = larger(gm, h[f]);
         }
       }
     }

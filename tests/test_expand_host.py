@@ -30,11 +30,18 @@ def test_expansion_accuracy(dp, tmp_path):
                     os.path.join(ROOT, "tests", "native", "expand_check.cpp"),
                     os.path.join(csrc, "expand.cpp"), os.path.join(csrc, "model.cpp"), "-o", exe],
                    check=True)
-    bad = dp.model.random_model("cu", seed=1000)
-    bad["emb_params"] = bad["emb_params"].copy()
-    bad["emb_params"][0, 3] = np.nan
+    def poisoned(at, value):
+        m = dp.model.random_model("cu", seed=1000)
+        m["emb_params"] = m["emb_params"].copy()
+        m["emb_params"][0, at] = value
+        return m
+
+    # a first-layer weight (every feature), one feature's last-layer bias (not
+    # the last feature) and weight
+    bad = [(poisoned(at, value), None, 0)
+           for at in (3, -7, -150) for value in (np.nan, np.inf, -np.inf)]
     cases = [("water", 0.25, 1), ("cu", 1.0, 1), ("water", 1.0, 2), ("hea", 1.0, 2),
-             ("water", 2.5, 4), ("water", 30.0, 0), (bad, None, 0)]
+             ("water", 2.5, 4), ("water", 30.0, 0)] + bad
     paths = []
     for k, (kind, scale, _) in enumerate(cases):
         m = kind if scale is None else scaled(dp, kind, scale)
