@@ -6,7 +6,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
-#include <system_error>
+#include <exception>
 #include <thread>
 
 #include "model.h"
@@ -56,22 +56,30 @@ void to_products(ld* c, int n, int S, int F) {
       }
 }
 
-// f(0) .. f(n - 1) over the host's cores (up to 8).
+// f(0) .. f(n - 1) over the host's cores (up to 8). What an f throws ends the
+// others' work too and is thrown again once every thread has.
 template <class Fn>
 void parallel(int n, Fn&& f) {
   std::atomic<int> next{0};
+  std::atomic<bool> failed{false};
+  std::exception_ptr error;  // written by the thread that sets failed
   auto work = [&]() {
-    for (int k = next++; k < n; k = next++) f(k);
+    try {
+      for (int k = next++; k < n && !failed; k = next++) f(k);
+    } catch (...) {
+      if (!failed.exchange(true)) error = std::current_exception();
+    }
   };
   std::vector<std::thread> pool;
   try {
     pool.reserve(7);
     for (int q = 1; q < std::min(n, 8); ++q) pool.emplace_back(work);
-  } catch (const std::system_error&) {
+  } catch (const std::exception&) {
     // fewer threads than asked for: the rest of the work stays here
   }
   work();
   for (auto& t : pool) t.join();
+  if (error) std::rethrow_exception(error);
 }
 
 // Chebyshev coefficients [n][L3] of the nets of `pairs` from n nodes (even),

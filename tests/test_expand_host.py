@@ -22,14 +22,23 @@ def scaled(dp, kind, scale):
     return m
 
 
-@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not found")
-def test_expansion_accuracy(dp, tmp_path):
-    exe = str(tmp_path / "expand_check")
+def build(tmp_path, name):
+    """tests/native/<name>.cpp with the expansion's host side."""
+    exe = str(tmp_path / name)
     csrc = os.path.join(PKG_DIR, "csrc")
     subprocess.run([HIPCC, "-O2", "-std=c++17", "--offload-arch=gfx950", "-w",
-                    os.path.join(ROOT, "tests", "native", "expand_check.cpp"),
+                    os.path.join(ROOT, "tests", "native", name + ".cpp"),
                     os.path.join(csrc, "expand.cpp"), os.path.join(csrc, "model.cpp"), "-o", exe],
                    check=True)
+    return exe
+
+
+needs_hipcc = pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not found")
+
+
+@needs_hipcc
+def test_expansion_accuracy(dp, tmp_path):
+    exe = build(tmp_path, "expand_check")
     def poisoned(at, value):
         m = dp.model.random_model("cu", seed=1000)
         m["emb_params"] = m["emb_params"].copy()
@@ -62,3 +71,14 @@ def test_expansion_accuracy(dp, tmp_path):
         assert eg <= 64 * groups * 2.0 ** -53 * gm, line
         assert ed <= (64 * groups) ** 2 * 2.0 ** -53 * gm * max(scale, 1.0) / 4, line
         assert f[5] == "0", line
+
+
+@needs_hipcc
+def test_expansion_out_of_memory(dp, tmp_path):
+    """An allocation that fails in any of the build's threads, or while they
+    are made, reaches the caller as an exception."""
+    exe = build(tmp_path, "expand_memory_check")
+    path = dp.model.write_model(str(tmp_path / "m.bin"), dp.model.random_model("cu", seed=1000))
+    r = subprocess.run([exe, path], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr
+    assert r.stdout.split()[0] == "ok" and int(r.stdout.split()[1]) > 10, r.stdout
