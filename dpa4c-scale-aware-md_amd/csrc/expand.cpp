@@ -84,7 +84,7 @@ void parallel(int n, Fn&& f) {
 
 // Chebyshev coefficients [n][L3] of the nets of `pairs` from n nodes (even),
 // and per pair the number of terms (a multiple of 16, 0 if none will do) past
-// which the magnitudes of every feature's coefficients sum to less than 2^-55
+// which the magnitudes of every feature's coefficients sum to at most 2^-55
 // of the largest feature: below the rounding of the sum itself, and small
 // enough that the derivative's truncation stays below its rounding too.
 void coefficients(const ModelHost& m, const std::vector<int>& pairs, int n,
@@ -126,7 +126,7 @@ void coefficients(const ModelHost& m, const std::vector<int>& pairs, int n,
   });
   for (int q = 0; q < np; ++q) {
     const int p = pairs[q];
-    ld gmax = 1.0L;
+    ld gmax = 0.0L;
     for (size_t k = 0; k < (size_t)n * F; ++k)
       gmax = std::max(gmax, std::fabs(val[(size_t)q * n * F + k]));
     terms[p] = 0;
@@ -135,7 +135,7 @@ void coefficients(const ModelHost& m, const std::vector<int>& pairs, int n,
       ld a = 0.0L;
       for (int f = 0; f < F; ++f) a = std::max(a, std::fabs(coef[p][(size_t)k * F + f]));
       tail += a;
-      if (!(tail < gmax * 0x1p-55L)) break;
+      if (tail > gmax * 0x1p-55L) break;
       if (k % 16 == 0 && k <= std::min(n - 16, kExpandMaxTerms)) terms[p] = k;
     }
   }

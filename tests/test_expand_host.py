@@ -49,6 +49,10 @@ def test_expansion_accuracy(dp, tmp_path):
     # the last feature) and weight
     bad = [(poisoned(at, value), None, 0)
            for at in (3, -7, -150) for value in (np.nan, np.inf, -np.inf)]
+    # features of 1e-6 at most: accuracy relative to them, not to one
+    small = dp.model.random_model("cu", seed=1000)
+    small["emb_params"] = small["emb_params"] * 1e-6
+    bad.append((small, None, 1))
     cases = [("water", 0.25, 1), ("cu", 1.0, 1), ("water", 1.0, 2), ("hea", 1.0, 2),
              ("water", 2.5, 4), ("water", 30.0, 0)] + bad
     paths = []
@@ -69,7 +73,7 @@ def test_expansion_accuracy(dp, tmp_path):
         # 2^-53 a few times; slopes: factors up to (term index) times the
         # slope in x near the ends, in units where x spans the range
         assert eg <= 64 * groups * 2.0 ** -53 * gm, line
-        assert ed <= (64 * groups) ** 2 * 2.0 ** -53 * gm * max(scale, 1.0) / 4, line
+        assert ed <= (64 * groups) ** 2 * 2.0 ** -53 * gm * max(scale or 1.0, 1.0) / 4, line
         assert f[5] == "0", line
 
 
