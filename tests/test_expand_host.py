@@ -86,3 +86,16 @@ def test_expansion_out_of_memory(dp, tmp_path):
     r = subprocess.run([exe, path], capture_output=True, text=True, timeout=100)
     assert r.returncode == 0, r.stderr
     assert r.stdout.split()[0] == "ok" and int(r.stdout.split()[1]) > 10, r.stdout
+
+
+@needs_hipcc
+def test_steep_nets_are_found_early(dp, tmp_path):
+    """A model whose nets have no expansion is known as such sooner than one
+    that has is built (it took four times as long when every net was tried with
+    every number of nodes); half as long again allows for a busy machine."""
+    exe = build(tmp_path, "expand_check")
+    paths = [dp.model.write_model(str(tmp_path / f"m{s}.bin"), scaled(dp, "hea", s)) for s in (1.0, 30.0)]
+    r = subprocess.run([exe] + paths, check=True, capture_output=True, text=True)
+    assert r.stdout.splitlines()[1] == "none"
+    flat, steep = (float(t) for t in r.stderr.split())
+    assert steep <= 1.5 * flat, (flat, steep)
