@@ -29,14 +29,15 @@ STAGE_ATOM_ENERGY, STAGE_EDGE_GRAD, STAGE_DEDD, STAGE_EXT_TYPE = 4, 5, 6, 7
 STAGE_C4_MOMENTS, STAGE_C4_COTANGENTS = 8, 9
 PREC_FP64, PREC_MIXED, PREC_MODEL = 0, 1, -1
 MODEL_SE_E2_A, MODEL_DPA4C = 0, 1
+FIT_NONE, FIT_FEW, FIT_PLAIN, FIT_FUSED = 0, 1, 2, 3
 
 EXPORTED = ("dp_create", "dp_destroy", "dp_get_info", "dp_last_error", "dp_compute",
             "dp_compute_nlist", "dp_compute_device", "dp_compute_device_async",
             "dp_compute_device_noalloc", "dp_sync",
             "dp_graph_stats", "dp_compute_canonical_graph_device", "dp_compute_edges_device",
             "dp_compute_edges_device_f32",
-            "dp_debug_copy", "dp_debug_keep", "dp_debug_fused_rows", "dp_stage_times",
-            "dp_device_bytes")
+            "dp_debug_copy", "dp_debug_keep", "dp_debug_fused_rows", "dp_debug_few_rows",
+            "dp_debug_fitting_form", "dp_stage_times", "dp_device_bytes")
 
 
 class DeepmdException(RuntimeError):
@@ -80,6 +81,8 @@ def lib():
         L.dp_debug_copy.restype = C.c_long
         L.dp_debug_keep.argtypes = [P, I]
         L.dp_debug_fused_rows.argtypes = [P, I]
+        L.dp_debug_few_rows.argtypes = [P, I]
+        L.dp_debug_fitting_form.argtypes = [P]
         L.dp_stage_times.argtypes = [P, I, P, I, P, C.c_size_t]
         L.dp_device_bytes.argtypes = [P]
         L.dp_device_bytes.restype = C.c_size_t
@@ -283,6 +286,16 @@ class DeepPot:
         """fp64 se_e2_a: use the fused dE/dD -> dE/dT kernel when every atom
         type has at least `rows` atoms (0: always; dp_debug_fused_rows)."""
         self._check(lib().dp_debug_fused_rows(self._h, int(rows)))
+
+    def set_few_rows(self, rows):
+        """se_e2_a: use the few-atoms fitting kernels up to `rows` atoms in all
+        (0: never; negative: the library's rule; dp_debug_few_rows)."""
+        self._check(lib().dp_debug_few_rows(self._h, int(rows)))
+
+    def fitting_form(self) -> int:
+        """FIT_FEW, FIT_PLAIN or FIT_FUSED: the fitting form of the last
+        evaluation (dp_debug_fitting_form)."""
+        return int(lib().dp_debug_fitting_form(self._h))
 
     def enable_stage_timing(self, on=True):
         times = (C.c_double * 16)()

@@ -171,6 +171,10 @@ struct dp_model {
   // dp_debug_fused_rows: smallest type (rows) for which the fp64 fitting uses
   // the fused dE/dD -> dE/dT kernel
   int fused_ddt_rows = 12288;
+  // dp_debug_few_rows: most atoms for which the fitting stage uses the few-atoms
+  // kernels (negative: few_rows())
+  int few_max = -1;
+  int fit_form = DP_FIT_NONE;  // of the last evaluation
   bool dd_valid = false;  // dE/dD of the last evaluation is in dD
   // stage timers
   bool timing = false;
@@ -569,14 +573,17 @@ void run_model_t(dp_model* M, hipStream_t st, int nloc, int nall, const int* d_n
     if (rows > 0) min_rows = std::min(min_rows, rows);
   }
   // few atoms in all: every type's chain in one set of latency-bound kernels
-  // (fit_few.hip); dp_debug_fused_rows(0) keeps the general kernels
+  // (fit_few.hip); dp_debug_fused_rows(0) and dp_debug_few_rows(0) keep the
+  // general kernels
   int present = 0;
   for (int t = 0; t < nt; ++t) present += M->type_off[t + 1] > M->type_off[t];
-  const bool few = d_from_t && nb <= few_rows(present, f32) && M->fused_ddt_rows > 0 &&
+  const int most_few = M->few_max >= 0 ? M->few_max : few_rows(present, f32);
+  const bool few = d_from_t && nb <= most_few && M->fused_ddt_rows > 0 &&
                    few_lds_bytes(nb, m.fit[0], sizeof(E)) <= 64 * 1024;
   const bool fused_ddt =
       d_from_t && !few && (f32 ? M->fitf_off[0][0][1] >= 0
                        : ddt_supported(m.fit[0], L3, axis) && min_rows >= M->fused_ddt_rows);
+  M->fit_form = few ? DP_FIT_FEW : fused_ddt ? DP_FIT_FUSED : DP_FIT_PLAIN;
   E* dD = ((!fused_ddt && !few) || M->keep_edge_grad) ? need<E>(M, M->dD, (size_t)std::max(nb, 1) * Dn)
                                             : nullptr;
   E* dT = need<E>(M, M->dT, (size_t)nloc * 4 * L3);
@@ -2004,5 +2011,13 @@ int dp_debug_fused_rows(dp_model* M, int rows) {
   M->fused_ddt_rows = rows;
   return DP_OK;
 }
+
+int dp_debug_few_rows(dp_model* M, int rows) {
+  if (!M) return DP_ERR_ARG;
+  M->few_max = rows;
+  return DP_OK;
+}
+
+int dp_debug_fitting_form(const dp_model* M) { return M ? M->fit_form : DP_ERR_ARG; }
 
 }  // extern "C"

@@ -313,9 +313,22 @@ int dp_debug_keep(dp_model* model, int keep);
  * few atoms per type. Systems of a few hundred to a few thousand atoms in all
  * run a set of kernels of their own (both precisions); rows == 0 switches
  * those off too. All forms give the same results to rounding. No
- * counterpart in the reference: a parity-test hook, so that both forms are
+ * counterpart in the reference: a parity-test hook, so that each form is
  * checked at the sizes the oracle evaluates. */
 int dp_debug_fused_rows(dp_model* model, int rows);
+
+/* se_e2_a: systems of at most `rows` atoms run the few-atoms fitting kernels
+ * (0: none, the forms above then apply to small systems too; negative, the
+ * default: the library's own rule). dp_debug_fitting_form names the form that the
+ * last evaluation ran. No counterparts in the reference: parity-test hooks. */
+enum {
+  DP_FIT_NONE = 0,  /* no se_e2_a evaluation yet */
+  DP_FIT_FEW = 1,   /* the few-atoms kernels */
+  DP_FIT_PLAIN = 2, /* dE/dD = dZ0 W0^T stored, then the dE/dT pass */
+  DP_FIT_FUSED = 3  /* the fused input-gradient kernel */
+};
+int dp_debug_few_rows(dp_model* model, int rows);
+int dp_debug_fitting_form(const dp_model* model);
 
 /* Per-stage GPU time in milliseconds (hipEvent pairs) of the last synchronous
  * evaluation, or the mean over the evaluations queued by

@@ -65,7 +65,8 @@ CASES = {"water192": water192, "cu864": cu_small, "hea1024": hea_small,
 # overrides)
 FALLBACK_SHAPES = {
     # F0 != 240 with axis 16: D formed inside the first GEMM, dE/dD as a
-    # plain product of the library's GEMM, then the axis-16 dE/dT kernel
+    # plain product of the library's GEMM, then the axis-16 dE/dT kernel (with
+    # the few-atoms kernels switched off: by default a system this small runs them)
     "water_f160": ("water192", dict(fit=[160, 160, 160])),
     # axis != 16: D stored by the descriptor kernel, the first layer reads it,
     # dE/dD plain, then the any-axis dE/dT kernel

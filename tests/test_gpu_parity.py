@@ -16,7 +16,24 @@ F_TOL = 1e-8    # eV/A
 V_TOL = 1e-8    # eV
 
 
-def _run(dp, orc, case, keep=False, fused=False):
+# the fitting stage's three forms, each selectable at every size: the few-atoms
+# kernels (what systems this small run by default), the plain product dE/dD with
+# the dE/dT pass, and the fused dE/dD -> dE/dT kernel
+FORMS = ["few", "plain_dD", "fused_dDdT"]
+
+
+def select_form(pot, form):
+    pot.set_few_rows(1 << 30 if form == "few" else 0)
+    if form == "fused_dDdT":
+        pot.set_fused_rows(0)
+
+
+def assert_form(dp, pot, form):
+    assert pot.fitting_form() == {"few": dp.FIT_FEW, "plain_dD": dp.FIT_PLAIN,
+                                  "fused_dDdT": dp.FIT_FUSED}[form]
+
+
+def _run(dp, orc, case, keep=False, form="few"):
     (coord, atype, box), m = CASES[case]()
     mb = model_bytes(m)
     O = orc.Oracle(mb)
@@ -24,11 +41,10 @@ def _run(dp, orc, case, keep=False, fused=False):
     pot = dp.DeepPot(file_content=mb)
     if keep:
         pot.keep_stages(True)
-    if fused:
-        # the fused dE/dD -> dE/dT kernel at this size too (by default a
-        # system this small takes the plain product and the dE/dT pass)
-        pot.set_fused_rows(0)
+    if form != "few":
+        select_form(pot, form)
     e, f, v, ae, av = pot.compute(coord, atype, box, atomic=True)
+    assert_form(dp, pot, form)
     return O, ref, pot, (e, f, v, ae, av), (coord, atype, box)
 
 
@@ -46,10 +62,10 @@ def test_nlist_bit_exact(dp, orc, case):
     assert np.array_equal(nl, ref["nlist"])
 
 
-@pytest.mark.parametrize("fused", [False, True], ids=["plain_dD", "fused_dDdT"])
+@pytest.mark.parametrize("form", FORMS)
 @pytest.mark.parametrize("case", list(CASES))
-def test_energy_force_virial(dp, orc, case, fused):
-    O, ref, pot, (e, f, v, ae, av), (coord, atype, box) = _run(dp, orc, case, fused=fused)
+def test_energy_force_virial(dp, orc, case, form):
+    O, ref, pot, (e, f, v, ae, av), (coord, atype, box) = _run(dp, orc, case, form=form)
     n = len(atype)
     assert abs(e - ref["energy"]) / n <= E_TOL
     assert np.abs(ae - ref["atom_energy"]).max() <= E_TOL
@@ -58,11 +74,10 @@ def test_energy_force_virial(dp, orc, case, fused):
     assert np.abs(av - ref["atom_virial"]).max() <= V_TOL
 
 
-@pytest.mark.parametrize("fused", [False, True], ids=["plain_dD", "fused_dDdT"])
+@pytest.mark.parametrize("form", FORMS)
 @pytest.mark.parametrize("case", ["water192", "cu864"])
-def test_stage_parity(dp, orc, case, fused):
-    O, ref, pot, (e, f, v, ae, av), (coord, atype, box) = _run(dp, orc, case, keep=True,
-                                                                fused=fused)
+def test_stage_parity(dp, orc, case, form):
+    O, ref, pot, (e, f, v, ae, av), (coord, atype, box) = _run(dp, orc, case, keep=True, form=form)
     n = len(atype)
     d = pot.stage(dp.STAGE_DESCRPT, np.float64, (n, O.ndescrpt))
     np.testing.assert_allclose(d, ref["descrpt"], rtol=0, atol=1e-12)
@@ -72,8 +87,7 @@ def test_stage_parity(dp, orc, case, fused):
     np.testing.assert_allclose(eg, ref["edge_grad"], rtol=0, atol=1e-11)
     # keeping the edge gradients changes no output
     pot2 = dp.DeepPot(file_content=model_bytes(CASES[case]()[1]))
-    if fused:
-        pot2.set_fused_rows(0)
+    select_form(pot2, form)
     e2, f2, v2, ae2, av2 = pot2.compute(coord, atype, box, atomic=True)
     assert e2 == e and np.array_equal(f2, f) and np.array_equal(v2, v)
     assert np.array_equal(av2, av)
@@ -300,12 +314,14 @@ def test_fitting_shapes(dp, orc, fit):
     assert np.abs(av - ref["atom_virial"]).max() <= V_TOL
 
 
+@pytest.mark.parametrize("few", [False, True])
 @pytest.mark.parametrize("name", list(FALLBACK_SHAPES))
 @pytest.mark.parametrize("mixed", [False, True])
-def test_fitting_fallback_shapes(dp, orc, name, mixed):
+def test_fitting_fallback_shapes(dp, orc, name, mixed, few):
     """Fitting shapes the fused dE/dD -> dE/dT kernels do not cover (first
-    fitting layer other than 240 wide, or axis other than 16): every output
-    against the oracle, in fp64 to the fp64 bar and in mixed precision to the
+    fitting layer other than 240 wide, or axis other than 16), on the general
+    kernels and where the library's rule takes the few-atoms kernels (axis 16)
+    on those: every output against the oracle, in fp64 to the fp64 bar and in mixed precision to the
     reference's mixed-precision limits; the library's own kernels only (no
     vendor BLAS is linked)."""
     from test_gpu_mixed import _check as mixed_check, _volume
@@ -313,8 +329,11 @@ def test_fitting_fallback_shapes(dp, orc, name, mixed):
     mb = model_bytes(m)
     ref = orc.Oracle(mb).compute(coord, atype, box)
     pot = dp.DeepPot(file_content=mb, precision=dp.PREC_MIXED if mixed else dp.PREC_FP64)
+    if not few:
+        pot.set_few_rows(0)
     got = pot.compute(coord, atype, box, atomic=True)
     n = len(atype)
+    assert pot.fitting_form() == (dp.FIT_FEW if few and m["axis"] == 16 else dp.FIT_PLAIN)
     if mixed:
         mixed_check(n, _volume(box), got, ref, f"{name} mixed")
         return

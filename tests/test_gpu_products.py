@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from cases import CASES, model_bytes
-from test_gpu_parity import E_TOL, F_TOL, V_TOL
+from test_gpu_parity import E_TOL, F_TOL, V_TOL, assert_form
 
 pytestmark = pytest.mark.gpu
 
@@ -29,6 +29,7 @@ def test_products(dp, orc, case, cells, drop, fused):
     if fused:
         pot.set_fused_rows(0)
     e, f, v, ae, av = pot.compute(coord, atype, box, atomic=True)
+    assert_form(dp, pot, "fused_dDdT" if fused else "plain_dD")
     assert abs(e - ref["energy"]) / n <= E_TOL
     assert np.abs(ae - ref["atom_energy"]).max() <= E_TOL
     assert np.abs(f - ref["force"]).max() <= F_TOL
