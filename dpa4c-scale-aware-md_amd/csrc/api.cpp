@@ -33,6 +33,7 @@
 
 #include "../../include/dp_amd.h"
 #include "expand.h"
+#include "fit_plan.h"
 #include "fixed.h"
 #include "kernels.h"
 #include "model.h"
@@ -435,21 +436,14 @@ void fit_types(dp_model* M, hipStream_t st, int nb, int Fmax, bool d_from_t, boo
   constexpr bool f32 = sizeof(E) == 4;
   const ModelHost& m = M->host;
   const int nt = m.ntypes, L3 = m.emb[2], Dn = L3 * m.axis;
-  int active = 0;
-  size_t ws_need = 0, ws_off = 0, ddt_need = 0, ddt_off = 0;
+  int active = 0, rows_of[kMaxTypes] = {0};
   for (int t = 0; t < nt; ++t) {
-    const int rows = M->type_off[t + 1] - M->type_off[t];
-    active += rows > 0;
-    const int sp = rows > 0 ? fit_splits(rows, m.fit[0], Dn, M->ncu, f32) : 1;
-    if (sp > 1) ws_need += (size_t)sp * rows * m.fit[0];
-    const int ds = (fused_ddt && rows > 0) ? ddt_splits(rows, L3, M->ncu) : 1;
-    if (ds > 1) ddt_need += (size_t)(ds + 1) * rows * 64;
+    rows_of[t] = M->type_off[t + 1] - M->type_off[t];
+    active += rows_of[t] > 0;
   }
-  // the fused input-gradient kernel's split partials, one region per type
-  double* ddt_ws = ddt_need ? need<double>(M, M->ddt_ws, ddt_need) : nullptr;
-  // split-K slices of the first layer, one region per type (the chains run
-  // concurrently)
-  E* split_ws = ws_need ? need<E>(M, M->split_ws, ws_need) : nullptr;
+  const FitPlan<kMaxTypes> plan = fit_plan(rows_of, m.fit[0], Dn, L3, M->ncu, f32, fused_ddt);
+  double* ddt_ws = plan.dws ? need<double>(M, M->ddt_ws, plan.dws) : nullptr;
+  E* split_ws = plan.ws ? need<E>(M, M->split_ws, plan.ws) : nullptr;
   const bool fork = active > 1 && !M->arena_on;
   // With the plain dE/dD product (few rows per type) the type with the most
   // rows stays on the evaluation stream, enqueued last, and only the others
@@ -504,9 +498,8 @@ void fit_types(dp_model* M, hipStream_t st, int nb, int Fmax, bool d_from_t, boo
     const size_t r0 = (size_t)M->type_off[t];
     const size_t slab = (size_t)std::max(nb, 1) * Fmax;
     FitBufs<E> fb{};
-    fb.split = fit_splits(rows, m.fit[0], Dn, M->ncu, f32);
-    if (fb.split > 1) fb.ws = split_ws + ws_off;
-    ws_off += (size_t)fb.split * rows * m.fit[0];
+    fb.split = plan.split[t];
+    if (fb.split > 1) fb.ws = split_ws + plan.ws_at[t];
     E* base = fitb;
     E** slots[6] = {&fb.H0, &fb.T1, &fb.H1, &fb.dZa, &fb.dZb, &fb.dH};
     // slab q holds [rows][F] of every type back to back; F <= Fmax. Slab 6
@@ -524,9 +517,8 @@ void fit_types(dp_model* M, hipStream_t st, int nb, int Fmax, bool d_from_t, boo
       ddt.dT = dT;
       ddt.dD = dD ? dD + r0 * Dn : nullptr;
       ddt.ncu = M->ncu;
-      ddt.nsplit = ddt_splits(rows, L3, M->ncu);
-      ddt.ws = ddt.nsplit > 1 ? ddt_ws + ddt_off : nullptr;
-      if (ddt.nsplit > 1) ddt_off += (size_t)(ddt.nsplit + 1) * rows * 64;
+      ddt.nsplit = plan.dsplit[t];
+      ddt.ws = ddt.nsplit > 1 ? ddt_ws + plan.dws_at[t] : nullptr;
     }
     launch_fitting(fst, net, rows, d_from_t ? nullptr : D + r0 * Dn,
                    d_from_t ? Tt + r0 * 4 : nullptr, 4L * nb, L3, fb, dD ? dD + r0 * Dn : nullptr,

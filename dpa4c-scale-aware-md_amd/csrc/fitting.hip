@@ -16,6 +16,7 @@
 
 #include "bf16x3.h"
 #include "fastmath.h"
+#include "fit_plan.h"
 #include "kernels.h"
 
 namespace dpamd {
@@ -566,20 +567,6 @@ __global__ __launch_bounds__(256) void k_splitk_tanh(int M, int N, int split,
   }
 #pragma unroll
   for (int j = 0; j < 4; ++j) C[o + j] = th[j];
-}
-
-// K slices for the first fitting layer: split only when the row blocks alone
-// leave the device short of work, and keep at least 8 K chunks of 16 per
-// slice. fp64: fewer than two blocks per compute unit (whole evaluation of
-// 12,288 water atoms 798 us, against 823 with a target of four; 24,000 atoms
-// 1,392 against 1,406; 3,993 and 98,304 atoms equal). fp32: fewer than four.
-int fit_splits(int rows, int N, int K, int ncu, bool f32) {
-  const int cols = N % 128 == 0 ? N / 128 : N % 80 == 0 ? N / 80 : N % 64 == 0 ? N / 64 : N / 16;
-  const long blocks = (long)cols * ((rows + 63) / 64);
-  const int nk = K / 16;
-  int split = 1;
-  while (blocks * split < (f32 ? 4L : 2L) * ncu && nk / (2 * split) >= 8) split *= 2;
-  return split;
 }
 
 // Energy head, second half: e = sum of the row's column-block partials of
@@ -1325,28 +1312,6 @@ void launch_fitting(hipStream_t st, const FitNet<T>& net, int rows, const T* D, 
 }
 
 bool ddt_supported(int K, int L3, int axis) { return K == 240 && axis == 16 && L3 >= 16 && L3 <= 128; }
-
-// Block shape of the fused kernel for a type of `rows` rows: eight waves (128
-// rows) when that gives every compute unit two blocks; four (64 rows) when
-// it gives one; otherwise eight waves with the column groups split over
-// blockIdx.y, enough ways to give every compute unit a block (at most one
-// way per 16 groups a >= 16). Returns the split count; *waves the shape.
-static int ddt_shape(int rows, int L3, int ncu, int* waves) {
-  const int nb8 = (rows + 127) / 128;
-  *waves = 8;
-  if (nb8 >= 2 * ncu) return 1;
-  if (nb8 >= ncu) {
-    *waves = 4;
-    return 1;
-  }
-  const int smax = std::max(1, (L3 - 16) / 16);
-  return std::min(smax, (ncu + nb8 - 1) / nb8);
-}
-
-int ddt_splits(int rows, int L3, int ncu) {
-  int waves = 0;
-  return ddt_shape(rows, L3, ncu, &waves);
-}
 
 void launch_dDdT(hipStream_t st, int rows, int K, int L3, const double* dZ, const double* W0T,
                  const double* Tt, long ldt, int pos0, const int* items, double* dT, double* dD,

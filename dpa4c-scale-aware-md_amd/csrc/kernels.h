@@ -258,13 +258,11 @@ template <class T>
 struct FitBufs {
   T *H0, *T1, *H1, *dZa, *dZb, *dH;  // [rows][F] each
   double* epart;  // [rows][F2 / column tile] partial energies of the head
-  // first layer split over K into `split` slices (fit_splits) summed through
+  // first layer split over K into `split` slices (fit_plan.h) summed through
   // ws [split][rows][F0] when split > 1
   int split;
   T* ws;
 };
-// K slices fit_splits(rows, F0, Dn, compute units) for the first fitting layer
-int fit_splits(int rows, int N, int K, int ncu, bool f32);
 // The first layer reads its input either from D ([rows][L3*axis]) or, when
 // Tt is given (axis 16), forms D = T^T T[:, :16] on the fly from the
 // column-major copy of T (element (row, a, m) at Tt[a * ldt + 4 row + m]) and
@@ -283,12 +281,11 @@ struct FitDdt {
   void* dT;           // [atoms][4][L3] (the net's precision)
   void* dD;           // [rows][16 L3] when kept for inspection, else null
   int ncu;
-  // column-group splits (ddt_splits) and their workspace, (nsplit + 1) *
+  // column-group splits (fit_plan.h) and their workspace, (nsplit + 1) *
   // rows * 64 doubles (unused when nsplit == 1)
   int nsplit;
   double* ws;
 };
-int ddt_splits(int rows, int L3, int ncu);
 bool ddt_supported(int F0, int L3, int axis);
 void launch_dDdT(hipStream_t, int rows, int K, int L3, const double* dZ, const double* W0T,
                  const double* Tt, long ldt, int pos0, const int* items, double* dT, double* dD,

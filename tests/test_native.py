@@ -40,6 +40,22 @@ def test_library_links_no_vendor_blas(dp):
     assert not [ln for ln in needed if "blas" in ln.lower()], needed
 
 
+def test_fitting_workspace_regions(tmp_path):
+    """The first layer's K slices and the input gradient's partials of several
+    types lie in disjoint regions of their workspaces, also where only some of
+    the types are split."""
+    import shutil
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("hipcc not found")
+    exe = str(tmp_path / "fit_plan_check")
+    src = os.path.join(ROOT, "tests", "native", "fit_plan_check.cpp")
+    subprocess.run([hipcc, "-O2", "-std=c++17", "--offload-arch=gfx950", "-w", src, "-o", exe], check=True)
+    out = subprocess.run([exe], capture_output=True, text=True)
+    assert out.returncode == 0, out.stdout
+    assert out.stdout.split()[0] == "ok" and int(out.stdout.split()[1]) > 1000, out.stdout
+
+
 def test_bad_model_is_reported(dp):
     L = dp.lib()
     h = ctypes.c_void_p()
