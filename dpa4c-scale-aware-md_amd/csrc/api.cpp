@@ -238,6 +238,14 @@ T* need(dp_model* M, Buf& b, size_t count) {
   return static_cast<T*>(b.p);
 }
 
+// Bytes that one more buffer may take: what the static scratch has left, no
+// bound outside it.
+size_t room(const dp_model* M) {
+  if (!M->arena_on) return SIZE_MAX;
+  const size_t off = (M->arena_used + 255) & ~size_t(255);
+  return off < M->arena_cap ? M->arena_cap - off : 0;
+}
+
 struct ApiError {
   int code;
   std::string msg;
@@ -441,8 +449,12 @@ void fit_types(dp_model* M, hipStream_t st, int nb, int Fmax, bool d_from_t, boo
     rows_of[t] = M->type_off[t + 1] - M->type_off[t];
     active += rows_of[t] > 0;
   }
-  const FitPlan<kMaxTypes> plan = fit_plan(rows_of, m.fit[0], Dn, L3, M->ncu, f32, fused_ddt);
+  FitPlan<kMaxTypes> plan = fit_plan(rows_of, m.fit[0], Dn, L3, M->ncu, f32, fused_ddt);
   double* ddt_ws = plan.dws ? need<double>(M, M->ddt_ws, plan.dws) : nullptr;
+  // (the slices only cost memory for speed, and are the last buffer carved from
+  // the static scratch: there they take what is left)
+  if (plan.ws > room(M) / sizeof(E))
+    plan = fit_plan(rows_of, m.fit[0], Dn, L3, M->ncu, f32, fused_ddt, room(M) / sizeof(E));
   E* split_ws = plan.ws ? need<E>(M, M->split_ws, plan.ws) : nullptr;
   const bool fork = active > 1 && !M->arena_on;
   // With the plain dE/dD product (few rows per type) the type with the most
@@ -651,8 +663,9 @@ void run_model_t(dp_model* M, hipStream_t st, int nloc, int nall, const int* d_n
     // fp64: the forward saves the layer-2/3 activations for the backward;
     // mixed precision recomputes them there (no buffer)
     const size_t blk = 16 * (size_t)(M->el.L2P + M->el.L3P);
-    // (the no-allocation entry point carves it in either case, so that the
-    // systems it accepts do not depend on the model's weights)
+    // (the no-allocation entry point reserves it in either case, so that what it
+    // refuses for the size does not turn on whether the weights have an expansion:
+    // the other buffers that differ move that limit by a tenth)
     ea.act = f32 || (expand && !M->arena_on)
                  ? nullptr
                  : need<E>(M, M->act, (size_t)std::max(nloc, 1) * acc * blk);
@@ -684,6 +697,10 @@ void run_model_t(dp_model* M, hipStream_t st, int nloc, int nall, const int* d_n
     return acc;
   };
 
+  // (here, so that the fitting's slices are the last buffer)
+  double* partials =
+      need<double>(M, M->partials, (size_t)finalize_ev_blocks(ntarget, nloc, nb) * 10);
+  double* out10 = need<double>(M, M->out10, 10);
   ExpandArgs xa{};
   if (expand) expand_args(M, ea, xa);
   int nblk = expand ? xa.wave_off[nt] : block_table(embed_waves_fwd(M->el, f32));
@@ -779,9 +796,6 @@ void run_model_t(dp_model* M, hipStream_t st, int nloc, int nall, const int* d_n
   }
   // forces and atom virials, then energy and frame virial (both stages of the
   // reduction under the force timer)
-  double* partials =
-      need<double>(M, M->partials, (size_t)finalize_ev_blocks(ntarget, nloc, nb) * 10);
-  double* out10 = need<double>(M, M->out10, 10);
   launch_finalize_ev(st, ntarget, nloc, nb, nsec, static_cast<const int*>(M->ext_type.p), cpsec,
                      fs, vs, fsum, vsum, e_bucket, out.force, out.atom_virial, partials, out10, out.energy,
                      out.virial);

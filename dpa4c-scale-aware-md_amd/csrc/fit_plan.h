@@ -4,6 +4,7 @@
 
 #include <algorithm>
 #include <cstddef>
+#include <cstdint>
 
 namespace dpamd {
 
@@ -46,7 +47,8 @@ inline int ddt_splits(int rows, int L3, int ncu) {
 // type, in one workspace of ws elements) and, on the fused kernels, their
 // column-group partials [splits + 1][rows][64] (in one of dws doubles). The
 // types' chains run concurrently: every split type has a region of its own, the
-// others none.
+// others none. The slices take at most ws_max elements: the most slices any type
+// has are halved until they do.
 template <int NT>
 struct FitPlan {
   int split[NT], dsplit[NT];
@@ -55,17 +57,27 @@ struct FitPlan {
 };
 
 template <int NT>
-FitPlan<NT> fit_plan(const int (&rows)[NT], int F0, int K, int L3, int ncu, bool f32, bool fused) {
+FitPlan<NT> fit_plan(const int (&rows)[NT], int F0, int K, int L3, int ncu, bool f32, bool fused,
+                     size_t ws_max = SIZE_MAX) {
   FitPlan<NT> p;
   for (int t = 0; t < NT; ++t) {
     p.split[t] = rows[t] > 0 ? fit_splits(rows[t], F0, K, ncu, f32) : 1;
     p.dsplit[t] = fused && rows[t] > 0 ? ddt_splits(rows[t], L3, ncu) : 1;
-    p.ws_at[t] = p.ws;
     p.dws_at[t] = p.dws;
-    if (p.split[t] > 1) p.ws += (size_t)p.split[t] * rows[t] * F0;
     if (p.dsplit[t] > 1) p.dws += (size_t)(p.dsplit[t] + 1) * rows[t] * 64;
   }
-  return p;
+  for (;;) {
+    p.ws = 0;
+    int most = 1;
+    for (int t = 0; t < NT; ++t) {
+      p.ws_at[t] = p.ws;
+      if (p.split[t] > 1) p.ws += (size_t)p.split[t] * rows[t] * F0;
+      most = std::max(most, p.split[t]);
+    }
+    if (p.ws <= ws_max || most == 1) return p;
+    for (int t = 0; t < NT; ++t)
+      if (p.split[t] == most) p.split[t] /= 2;
+  }
 }
 
 }  // namespace dpamd

@@ -1,8 +1,8 @@
 // Workspace regions of the general fitting chains (csrc/fit_plan.h): over row
 // counts per type on both sides of every rule, in every order, a split type's
 // region must lie in the workspace and overlap no other's, and an unsplit type
-// must take none. Prints "ok" and the number of plans that mix split and unsplit
-// types.
+// must take none; and with less memory than the slices ask for, they must fit it.
+// Prints "ok" and the number of plans that mix split and unsplit types.
 #include <cstdio>
 #include <cstdlib>
 
@@ -36,6 +36,16 @@ int main() {
         }
         if (ws != p.ws || dws != p.dws) return std::printf("unused memory\n"), 1;
         mixed += split > 0 && whole > 0;
+        for (size_t most = p.ws; most > 0; most = most / 4 * 3) {
+          const FitPlan<NT> q = fit_plan(rows, 240, 1600, 100, 256, f32, fused, most);
+          bool less = q.dws == p.dws && q.ws <= most;
+          size_t end = 0;
+          for (int t = 0; t < NT; ++t) {
+            less = less && q.split[t] >= 1 && q.split[t] <= p.split[t] && q.ws_at[t] >= end;
+            if (q.split[t] > 1) end = q.ws_at[t] + (size_t)q.split[t] * rows[t] * 240;
+          }
+          if (!less || end > q.ws) return std::printf("slices in %zu elements\n", most), 1;
+        }
       }
   std::printf("ok %d\n", mixed);
   return 0;

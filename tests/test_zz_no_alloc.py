@@ -75,7 +75,8 @@ def test_noalloc_matches_device_entry_point_twice(dp, case):
     outside the fused kernels; a DPA4C-Nano model on the HEA pair), then the
     first again: each agrees with dp_compute_device. The saved fp64 embedding activations (16 (L2P +
     L3P) doubles per 16-slot tile: 295 KB per HEA atom, 221 KB per Cu atom)
-    bound what fits in 128 MiB; the mixed path saves none."""
+    bound what fits in 128 MiB, and are reserved also where the nets' expansion
+    saves none; the mixed path reserves none."""
     hip = importlib.import_module("dpamd.hip")
     if case == "water192":
         (coord, atype, box), m = CASES[case]()
@@ -135,10 +136,32 @@ def test_noalloc_allocates_no_device_memory(dp):
     assert pot.device_bytes() == bytes0
 
 
+def test_noalloc_takes_fewer_slices_for_want_of_memory(dp):
+    """A thin rod (two Cu cells wide, so 74 images of every atom) of 3,520
+    atoms in mixed precision with atom outputs fills the scratch but for less than
+    the fitting's K slices take elsewhere: the call runs with fewer of them, to
+    the rounding of fp32 sums in another order (the mixed-precision limits)."""
+    from test_gpu_mixed import _check as mixed_check, _volume
+    hip = importlib.import_module("dpamd.hip")
+    n, a, cells = 3520, 3.615, 220
+    base = np.array([[0, 0, 0], [.5, .5, 0], [.5, 0, .5], [0, .5, .5]])
+    grid = np.stack(np.meshgrid(np.arange(2), np.arange(2), np.arange(cells), indexing="ij"), -1)
+    coord = a * (grid.reshape(-1, 1, 3) + base).reshape(-1, 3)
+    coord = coord + 0.02 * np.random.default_rng(5).standard_normal(coord.shape)
+    box = np.diag([2 * a, 2 * a, cells * a]).reshape(9)
+    atype = np.zeros(n, np.int32)
+    pot = dp.DeepPot(file_content=model_bytes(CASES["cu864"]()[1]), precision=dp.PREC_MIXED)
+    got, ref = _both(hip, pot, (coord, atype, box))
+    ref = dict(zip(("energy", "force", "virial", "atom_energy", "atom_virial"), ref))
+    mixed_check(n, _volume(box), got, ref, "rod")
+
+
 def test_noalloc_rejects_system_beyond_scratch(dp):
-    """2048 Cu atoms need about 450 MB of saved activations, beyond the
-    128 MiB scratch: the call fails with a capacity error naming the limit,
-    and both entry points work on the handle afterwards."""
+    """2048 Cu atoms in fp64 are beyond the 128 MiB scratch, which reserves the
+    saved activations of the slot-by-slot embedding kernels (about 450 MB) whether
+    or not the model's nets have an expansion: the call fails with a capacity
+    error naming the limit, and both entry points work on the handle
+    afterwards."""
     hip = importlib.import_module("dpamd.hip")
     m = CASES["cu864"]()[1]
     coord, atype, box = dp.systems.fcc(4, 3.615, seed=4)
