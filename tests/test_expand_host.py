@@ -54,7 +54,7 @@ def test_expansion_accuracy(dp, tmp_path):
     small["emb_params"] = small["emb_params"] * 1e-6
     bad.append((small, None, 1))
     cases = [("water", 0.25, 1), ("cu", 1.0, 1), ("water", 1.0, 2), ("hea", 1.0, 2),
-             ("water", 2.5, 4), ("water", 30.0, 0)] + bad
+             ("water", 2.5, 4), ("hea", 2.5, 4), ("water", 30.0, 0)] + bad
     paths = []
     for k, (kind, scale, _) in enumerate(cases):
         m = kind if scale is None else scaled(dp, kind, scale)
