@@ -49,50 +49,6 @@ struct alignas(2 * sizeof(E)) Vec2 {
   E x, y;
 };
 
-// Basis values T_1..T_3, T_4, T_8, T_12, T_16, T_32, T_48 (v[1..9], v[0] = 1),
-// then T_64, T_128, T_192 for the groups in use.
-template <int H>
-constexpr int kNumBasis = 10 + (H > 1 ? 1 : 0) + (H > 2 ? 2 : 0);
-
-template <int H>
-__device__ __forceinline__ void basis_values(double x, double* v) {
-  v[0] = 1.0;
-  v[1] = x;
-  v[2] = fma(2.0 * x, x, -1.0);
-  v[3] = x * fma(4.0 * x, x, -3.0);
-  v[4] = fma(2.0 * v[2], v[2], -1.0);
-  v[5] = fma(2.0 * v[4], v[4], -1.0);
-  v[6] = v[4] * fma(4.0 * v[4], v[4], -3.0);
-  v[7] = fma(2.0 * v[5], v[5], -1.0);
-  v[8] = fma(2.0 * v[7], v[7], -1.0);
-  v[9] = v[7] * fma(4.0 * v[7], v[7], -3.0);
-  if constexpr (H > 1) v[10] = fma(2.0 * v[8], v[8], -1.0);
-  if constexpr (H > 2) {
-    v[11] = fma(2.0 * v[10], v[10], -1.0);
-    v[12] = v[10] * fma(4.0 * v[10], v[10], -3.0);
-  }
-}
-
-// ... and their derivatives in x
-template <int H>
-__device__ __forceinline__ void basis_slopes(double x, const double* v, double* d) {
-  d[0] = 0.0;
-  d[1] = 1.0;
-  d[2] = 4.0 * x;
-  d[3] = fma(12.0 * x, x, -3.0);
-  d[4] = 4.0 * v[2] * d[2];
-  d[5] = 4.0 * v[4] * d[4];
-  d[6] = fma(12.0 * v[4], v[4], -3.0) * d[4];
-  d[7] = 4.0 * v[5] * d[5];
-  d[8] = 4.0 * v[7] * d[7];
-  d[9] = fma(12.0 * v[7], v[7], -3.0) * d[7];
-  if constexpr (H > 1) d[10] = 4.0 * v[8] * d[8];
-  if constexpr (H > 2) {
-    d[11] = 4.0 * v[10] * d[10];
-    d[12] = fma(12.0 * v[10], v[10], -3.0) * d[10];
-  }
-}
-
 // Environment row of a slot (as env_value) and the expansion's y.
 __device__ __forceinline__ double env_row(const ExpandArgs& a, double d0, double d1, double d2,
                                           const double* avg, const double* isd, double* Rn) {

@@ -1,9 +1,10 @@
 // The embedding nets' expansion on the host (csrc/expand.cpp): for each model
 // file named on the command line, prints one line
-//   ok H max|G - sum C phi| max|G' - sum C phi'| max|G|
+//   ok H max|G - sum C phi| max|G' - sum C phi'| the same near the cutoff
+//   max|G| max|G'| (differences of the two layouts)
 // over distances from the range's end to the cutoff, with the coefficients
-// read back from both operand layouts, the basis evaluated in fp64 as the
-// kernels do and the net and its tangent in extended precision; or "none"
+// read back from both operand layouts, the basis from the kernels' own functions
+// in fp64 and the net and its tangent in extended precision; or "none"
 // when some net has no short enough expansion. The best of three builds' times,
 // in ms, goes to stderr, a line a model.
 #include <algorithm>
@@ -51,7 +52,7 @@ int main(int argc, char** argv) {
     }
     const int np = m.ntypes * m.ntypes, F = m.emb[2], N = 64 * e.H;
     const int NU2 = expand_nu2(F), NQ2 = expand_nq2(F);
-    double eg = 0, ed = 0, gm = 0;
+    double eg = 0, ed = 0, en = 0, gm = 0, dm = 0;
     int layouts = 0;
     for (int p = 0; p < np; ++p) {
       const double* cf = e.fwd.data() + p * expand_fwd_stride(e.H, F);
@@ -67,29 +68,18 @@ int main(int argc, char** argv) {
       const double avg = m.davg[4 * p], sd = m.dstd[4 * p];
       for (int s = 0; s <= 200; ++s) {
         const double y = s / 200.0;  // rmin sw / r: 0 at the cutoff, 1 at the range's end
-        // fp64 basis
-        const double iv = 1.0 / (1.0 + y), x = kExpandA * 2.0 * y * iv - kExpandB;
-        std::vector<double> T(N), D(N);
-        auto cheb = [&](int n, double* v, double* d) {
-          double a = 1, b = x, da = 0, db = 1;  // T_0, T_1 and slopes
-          if (n == 0) { *v = 1; *d = 0; return; }
-          for (int k = 1; k < n; ++k) {
-            const double c = 2 * x * b - a, dc = 2 * b + 2 * x * db - da;
-            a = b; b = c; da = db; db = dc;
-          }
-          *v = b; *d = db;
-        };
-        for (int k = 0; k < N; ++k) {
-          const int part[4] = {k / 64 * 64, k / 16 % 4 * 16, k / 4 % 4 * 4, k % 4};
-          double v = 1, d = 0;
-          for (int n : part) {
-            double t, dt;
-            cheb(n, &t, &dt);
-            d = d * t + v * dt;
-            v *= t;
-          }
-          T[k] = v;
-          D[k] = d;
+        // basis functions and slopes as the kernels form them
+        const double iv = 1.0 / (1.0 + y), x = fma(kExpandA * 2.0 * y, iv, -kExpandB);
+        const int H = e.H;
+        double v[kNumBasis<4>], sl[kNumBasis<4>];
+        if (H == 1) basis_values<1>(x, v), basis_slopes<1>(x, v, sl);
+        else if (H == 2) basis_values<2>(x, v), basis_slopes<2>(x, v, sl);
+        else basis_values<4>(x, v), basis_slopes<4>(x, v, sl);
+        double c[16], dc[16];
+        for (int k = 0; k < 16; ++k) {
+          const int l = k % 4, p4 = k / 4 ? 3 + k / 4 : 0;
+          c[k] = v[l] * v[p4];
+          dc[k] = fma(sl[l], v[p4], v[l] * sl[p4]);
         }
         // the net and its slope in extended precision
         std::vector<ld> h{((ld)y / (ld)kExpandRmin - avg) / sd}, t{1};
@@ -116,18 +106,28 @@ int main(int argc, char** argv) {
         }
         const double dxds = kExpandA * 2.0 * iv * iv * kExpandRmin * sd;
         for (int f = 0; f < F; ++f) {
+          // (sums of 16 terms, then over the blocks, as the backward)
           double g = 0, d = 0;
-          for (int k = 0; k < N; ++k) {
-            g += C[(size_t)k * F + f] * T[k];
-            d += C[(size_t)k * F + f] * D[k];
+          for (int k = 0; k < N; k += 16) {
+            double Y = 0, Yd = 0;
+            for (int q = 0; q < 16; ++q) {
+              Y = fma(C[(size_t)(k + q) * F + f], c[q], Y);
+              Yd = fma(C[(size_t)(k + q) * F + f], dc[q], Yd);
+            }
+            const int b = k / 16 % 4 ? 6 + k / 16 % 4 : 0, h64 = k / 64 ? 9 + k / 64 : 0;
+            const double w = v[b] * v[h64], dw = fma(sl[b], v[h64], v[b] * sl[h64]);
+            g = fma(w, Y, g);
+            d = fma(dw, Y, fma(w, Yd, d));
           }
           eg = larger(eg, g - h[f]);
           ed = larger(ed, d * dxds - t[f]);
           gm = larger(gm, h[f]);
+          dm = larger(dm, t[f]);
+          if (y <= 0.1) en = larger(en, d * dxds - t[f]);
         }
       }
     }
-    std::printf("ok %d %.3e %.3e %.3e %d\n", e.H, eg, ed, gm, layouts);
+    std::printf("ok %d %.3e %.3e %.3e %.3e %.3e %d\n", e.H, eg, ed, en, gm, dm, layouts);
   }
   return 0;
 }
