@@ -358,9 +358,9 @@ struct Outputs {
   double* atom_virial;  // device [ntarget][9] or null
 };
 
-// Everything after the neighbour list; ext/ext_type/nlist/nreal/mapping ready.
-// Arguments of the descriptor kernel for the current buckets: T (and D when
-// non-null) in bucket order from Tsec.
+// Arguments of the descriptor kernel for the current buckets: D (when non-null)
+// in bucket order from T, which it first forms from the sections' Tsec where the
+// forward has not.
 DescArgs desc_args(dp_model* M, void* Tt, void* D) {
   const ModelHost& m = M->host;
   DescArgs da{};
@@ -641,8 +641,6 @@ void run_model_t(dp_model* M, hipStream_t st, int nloc, int nall, const int* d_n
   ea.edge_grad = edge_grad;
   ea.facc = facc;
   ea.vacc = vacc;
-  ea.fs = fs;
-  ea.vs = vs;
   ea.cpsec = cpsec;
   // the fixed-point sums are cleared by the forward (no kernel of their own;
   // stores, not a memset, so the step can be captured in a graph); on the
@@ -1949,7 +1947,7 @@ long dp_debug_copy(dp_model* M, int stage, void* dst, size_t capacity) {
         if (M->kind == dp_model::kDpa4c)
           throw ApiError{DP_ERR_ARG, "the DPA4C path keeps its descriptor in registers"};
         if (M->host.axis == 16 && M->nbucket > 0) {
-          // not stored by the evaluation: form D from the saved Tsec
+          // not stored by the evaluation: form D from T
           void* Dp = need<char>(M, M->D, (size_t)M->nbucket * Dn * net_esize);
           launch_descriptor(nullptr, desc_args(M, M->Tt.p, Dp), net_esize == 4);
         }

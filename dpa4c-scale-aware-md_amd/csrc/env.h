@@ -125,7 +125,7 @@ __device__ __forceinline__ void edge_out(const EmbArgs& a, long e, int t, const 
     // would wrap silently in the integer sums
     const double gm = fmax(fabs(gv[0]), fmax(fabs(gv[1]), fabs(gv[2])));
     if (!(gm <= a.fix_gmax)) atomicOr(a.status, kStatusFixedRange);
-    unsigned long long* fa = a.facc + (long)a.fs * t;
+    unsigned long long* fa = a.facc + 3L * t;
     fixed_add(fa, gv[0]);
     fixed_add(fa + 1, gv[1]);
     fixed_add(fa + 2, gv[2]);
@@ -138,7 +138,7 @@ __device__ __forceinline__ void edge_out(const EmbArgs& a, long e, int t, const 
   } else if constexpr (AV) {
     const int c = grp - 1;
     const double gc = grp == 1 ? gv[0] : grp == 2 ? gv[1] : gv[2];
-    unsigned long long* va = a.vacc + (long)a.vs * t + 3 * c;
+    unsigned long long* va = a.vacc + 9L * t + 3 * c;
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
       const double v = -gc * d[q];
@@ -180,9 +180,9 @@ __device__ __forceinline__ void clear_fixed(const EmbArgs& a) {
   const long n = a.zero_count ? (long)*a.zero_count : a.zero_n;
   const long stride = (long)gridDim.x * blockDim.x;
   const long q0 = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  for (long q = q0; q < a.fs * n; q += stride) a.facc[q] = 0ull;
+  for (long q = q0; q < 3 * n; q += stride) a.facc[q] = 0ull;
   if (a.vacc)
-    for (long q = q0; q < a.vs * n; q += stride) a.vacc[q] = 0ull;
+    for (long q = q0; q < 9 * n; q += stride) a.vacc[q] = 0ull;
 }
 
 __device__ __forceinline__ int find_pair(const EmbArgs& a) {

@@ -1144,13 +1144,13 @@ static size_t ddt_lds_bytes(int K) {
 // epilogues each operand form is used with: the first layer (A from T) plain
 // or forward, the other forward layers forward or last-layer-with-head, the
 // transposed-B products plain or backward.
-template <class T, int NT, bool TRANSB, bool AT, int EPI>
+template <class T, int NT, bool BWD, bool AT, int EPI>
 static void gemm_launch(hipStream_t st, const GemmArgs<T>& a, dim3 grid) {
   if constexpr (sizeof(T) == 8) {
     hipLaunchKernelGGL((k_gemm_d<NT, AT, EPI>), grid, dim3(256), 0, st, a);
   } else if (a.Bf) {  // B pre-split: the bf16 three-piece kernel (B's orientation is in the fragments)
     hipLaunchKernelGGL((k_gemm3<NT, AT, EPI>), grid, dim3(256), 0, st, a);
-  } else if constexpr (TRANSB && EPI == 0) {
+  } else if constexpr (BWD && EPI == 0) {
     hipLaunchKernelGGL(k_gemm<NT>, grid, dim3(256), 0, st, a);
   } else {
     throw HipError{hipErrorInvalidValue, "fitting GEMM: no bf16 fragments of this layer"};
@@ -1158,17 +1158,17 @@ static void gemm_launch(hipStream_t st, const GemmArgs<T>& a, dim3 grid) {
   DPAMD_LAUNCH_CHECK();
 }
 
-template <class T, int NT, bool TRANSB, bool AT = false>
+template <class T, int NT, bool BWD, bool AT = false>
 static void gemm_nt(hipStream_t st, const GemmArgs<T>& a) {
   dim3 grid(a.N / (16 * NT), (a.M + 63) / 64, a.split > 1 ? a.split : 1);
-  if constexpr (TRANSB) {
-    if (a.epi == 0) return gemm_launch<T, NT, TRANSB, AT, 0>(st, a, grid);
-    if (a.epi == 2) return gemm_launch<T, NT, TRANSB, AT, 2>(st, a, grid);
+  if constexpr (BWD) {
+    if (a.epi == 0) return gemm_launch<T, NT, BWD, AT, 0>(st, a, grid);
+    if (a.epi == 2) return gemm_launch<T, NT, BWD, AT, 2>(st, a, grid);
   } else if constexpr (AT) {
-    if (a.epi == 1) return gemm_launch<T, NT, TRANSB, AT, 1>(st, a, grid);
+    if (a.epi == 1) return gemm_launch<T, NT, BWD, AT, 1>(st, a, grid);
   } else {
-    if (a.epi == 1) return gemm_launch<T, NT, TRANSB, AT, 1>(st, a, grid);
-    if (a.epi == 3) return gemm_launch<T, NT, TRANSB, AT, 3>(st, a, grid);
+    if (a.epi == 1) return gemm_launch<T, NT, BWD, AT, 1>(st, a, grid);
+    if (a.epi == 3) return gemm_launch<T, NT, BWD, AT, 3>(st, a, grid);
   }
   throw HipError{hipErrorInvalidValue, "fitting GEMM: epilogue not available for this operand form"};
 }
@@ -1189,20 +1189,20 @@ static int col_tiles(int M, int N) {
     if (tiles % k == 0 && (nt == 1 || rb * (tiles / k) >= kFullGrid)) nt = k;
   return nt;
 }
-template <bool TRANSB, class T>
+template <bool BWD, class T>
 static void gemm(hipStream_t st, const GemmArgs<T>& a) {
   if (a.M <= 0) return;
   switch (col_tiles<T>(a.M, a.N)) {
-    case 8: gemm_nt<T, 8, TRANSB>(st, a); break;
-    case 5: gemm_nt<T, 5, TRANSB>(st, a); break;
-    case 4: gemm_nt<T, 4, TRANSB>(st, a); break;
+    case 8: gemm_nt<T, 8, BWD>(st, a); break;
+    case 5: gemm_nt<T, 5, BWD>(st, a); break;
+    case 4: gemm_nt<T, 4, BWD>(st, a); break;
     case 3:
       if constexpr (sizeof(T) == 8) {
-        gemm_nt<T, 3, TRANSB>(st, a);
+        gemm_nt<T, 3, BWD>(st, a);
         break;
       }
       [[fallthrough]];
-    default: gemm_nt<T, 1, TRANSB>(st, a);
+    default: gemm_nt<T, 1, BWD>(st, a);
   }
 }
 

@@ -64,8 +64,8 @@ struct EmbArgs {
   // Backward outputs. Each slot's edge gradient goes to its centre's
   // section sums cpsec [nloc][ntypes][12] (force 3, frame virial 9, fp64)
   // and, in fixed point (fixed.h), to its neighbour's extended-atom slot j:
-  // facc [nall][fs] (three used) and, when non-null, vacc [nall][vs] (nine
-  // used) (launch_fold_fixed then moves ghost sums onto their owners). The forward clears both sums
+  // facc [nall][3] and, when non-null, vacc [nall][9] (launch_fold_fixed
+  // then moves ghost sums onto their owners). The forward clears both sums
   // at its end for the backward: zero_n atoms, or *zero_count when
   // zero_count is non-null.
   // edge_grad [nloc][nnei][3] is written only when non-null (kept for
@@ -73,7 +73,6 @@ struct EmbArgs {
   double* edge_grad;
   unsigned long long* facc;
   unsigned long long* vacc;
-  int fs, vs;
   double* cpsec;
   long zero_n;
   const int* zero_count;
@@ -155,7 +154,7 @@ struct DescArgs {
 };
 
 // Neighbour stage
-// also clears clear[0 .. nclear) and, when nall is given, sets *nall = nloc
+// (boxes without ghost images) also clears clear[0 .. nclear) and sets *nall = nloc
 void launch_wrap(hipStream_t, int nloc, const double* coord, const int* atype, const BoxParams&,
                  double* ext, int* ext_type, int* mapping, int nclear, int* clear, int* nall);
 // Ghost images in (shift, atom) order: wraps the atoms (ext, ext_type, mapping,
@@ -339,12 +338,14 @@ void launch_rev_count(hipStream_t, long nedge, int nnei, const int* nlist, const
                       int* count, int* rank);
 void launch_rev_fill(hipStream_t, long nedge, int nnei, const int* nlist, const int* mapping,
                      const int* off, const int* rank, int* rev);
-// Fixed-point sums src of extended atoms j in [j0, n) (force [.][fs], virial
-// [.][vs] or null, in src as in dst) added onto their owners mapping[j] in dst (integer atomics: order-independent); dst may be
+// Fixed-point sums src of extended atoms j in [j0, n) (rows of fs and vs words, in
+// src as in dst: three force values, and nine of the virial or null) added onto
+// their owners mapping[j] in dst (integer atomics: order-independent); dst may be
 // src when every owner lies below j0. n = *d_count when d_count is given (a
 // count on the device, at most cap), else cap; src_v / dst_v may be null.
 void launch_fold_fixed(hipStream_t, int j0, int cap, const int* d_count, const int* mapping,
-                       int fs, int vs, const unsigned long long* src_f, const unsigned long long* src_v,
+                       int fs, int vs, const unsigned long long* src_f,
+                       const unsigned long long* src_v,
                        unsigned long long* dst_f, unsigned long long* dst_v);
 // p[0 .. per * n) = 0 for 64-bit words, n = *d_count (at most cap) or cap
 void launch_zero_u64(hipStream_t, long cap, const int* d_count, int per, unsigned long long* p);
