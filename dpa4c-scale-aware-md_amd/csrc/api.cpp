@@ -50,9 +50,13 @@ struct Buf {
 // Atoms up to which the fitting stage takes the few-atoms kernels (fit_few.hip):
 // their time grows with the atoms of all types together, that of the general
 // chains with the launches per type. Queued steps, few / general kernels, us:
-// fp64 Cu 256 atoms 178 / 250, 864 262 / 271, 2916 503 / 375; water 192 180 /
-// 285, 1536 323 / 336, 3000 499 / 384; HEA 1024 303 / 431, 3456 639 / 569.
-// Mixed HEA 250 204 / 525, 2662 423 / 586, 5488 687 / 685.
+// fp64 Cu 256 atoms 136 / 199, 864 221 / 225, 1372 282 / 257; water 192 137 /
+// 236, 1029 271 / 280, 1536 284 / 287, 2187 411 / 340; HEA 1024 248 / 341, 2000
+// 387 / 399, 2662 503 / 460. Mixed Cu 864 181 / 212, 1372 228 / 226; water 1536
+// 231 / 278, 2187 321 / 312; HEA 1024 211 / 447, 4394 552 / 574, 5488 628 / 595.
+// They cross at about 930, 1560 and 2150 atoms (one, two, four types) in fp64 and
+// 1350, 2100 and 4800 mixed; the lines below are within 15 % of that but for four
+// types in fp64, where the stretch from 2150 to 2700 atoms costs up to 9 %.
 int few_rows(int types, bool f32) { return f32 ? 1200 * types : 300 + 600 * types; }
 
 enum Stage {
@@ -170,7 +174,15 @@ struct dp_model {
   bool keep_edge_grad = false;
   bool eg_valid = false;
   // dp_debug_fused_rows: smallest type (rows) for which the fp64 fitting uses
-  // the fused dE/dD -> dE/dT kernel
+  // the fused dE/dD -> dE/dT kernel. Queued steps, plain / fused, us (rows of the
+  // smallest type in brackets): Cu 8,788 755 / 848, 10,976 933 / 1047, 13,500 1036 /
+  // 1104, 16,384 1120 / 1072, 19,652 1381 / 1517, 23,328 1643 / 1719, 32,000 2111 /
+  // 2016, 42,592 2768 / 2753; water 12,288 (4,096) 796 / 943, 31,944 (10,648) 1849 /
+  // 1958, 41,472 (13,824) 2386 / 2387, 52,728 (17,576) 2952 / 3035, 65,856 (21,952)
+  // 3758 / 3654; HEA 27,648 (6,912) 2026 / 2127, 43,904 (10,976) equal, 54,000
+  // (13,500) 3819 / 3731. Below the line the plain product is always ahead, above
+  // 25,000 rows the fused kernel; between them it turns on how evenly the fused
+  // kernel's blocks of 64 or 128 rows fill the compute units.
   int fused_ddt_rows = 12288;
   // dp_debug_few_rows: most atoms for which the fitting stage uses the few-atoms
   // kernels (negative: few_rows())

@@ -764,7 +764,10 @@ namespace {
 // Blocks of four waves up to this many groups of four centres (half a group
 // per SIMD). Queued steps with blocks of one / four waves, us: water 192 atoms
 // 177 / 147, 1536 338 / 314, 3993 440 / 442, 12288 861 / 975; Cu 864 262 / 236,
-// 4000 461 / 462; HEA mixed 1024 262 / 232, 3456 489 / 528.
+// 4000 461 / 462; HEA mixed 1024 262 / 232, 3456 489 / 528. With four groups of
+// terms (a block's LDS then fills a compute unit) they cross a little lower, at
+// about 430: water 1536 351 / 343, 2187 383 / 420; HEA mixed 1024 291 / 241, 2000
+// 372 / 407, 2662 449 / 566.
 constexpr int kSharedGroups = 512;
 
 template <class K>
