@@ -42,6 +42,7 @@ PEAK_FP64_MFMA = 78.6e12   # FLOP/s, MI355X dense FP64 matrix
 PEAK_HBM = 8.0e12          # B/s
 PEAK_FP32_MFMA = 157.3e12  # FLOP/s, MI355X dense FP32 matrix
 PEAK_FP32_VALU = 157.3e12  # FLOP/s, MI355X FP32 vector
+FIT_PLAIN = 2              # dp_debug_fitting_form: dE/dD stored, then the dE/dT pass
 DT_FS = {0: 0.5, 1: 0.5, 2: 1.0, 3: 1.0, 4: 0.5}
 KIND = {0: "water", 1: "water", 2: "cu", 3: "hea", 4: "water"}
 # config 3 is specified in mixed precision (fp32 nets, fp64 env/force/virial)
@@ -55,15 +56,14 @@ WORKLOAD = {2: "cu131k FCC Cu 131,072 atoms, rcut 8, sel 138, 32-64-128/240x3",
 
 def flops_bytes(pot, n_real, nloc, mixed=False):
     """Algorithmic FLOPs / bytes of each stage for one step (real slots only;
-    padded slots are a per-(type, type) constant and not evaluated). The
-    descriptor arrays (section sums, T, dE/dD, dE/dT) are fp32 in mixed mode.
-    With one neighbour type the forward writes T itself and the descriptor
-    pass does not run, so it has no work of its own."""
+    padded slots are a per-(type, type) constant and not evaluated). T, dE/dD
+    and dE/dT are fp32 in mixed mode. The expanded nets' forward writes T
+    itself, so no descriptor pass runs. Call it after an evaluation: dE/dT has
+    a pass of its own only where the fitting ran the plain product dE/dD."""
     L1, L2, L3 = (pot.info.emb[k] for k in range(3))
     M2 = pot.info.axis
     F0, F1, F2 = (pot.info.fit[k] for k in range(3))
     Dn = L3 * M2
-    nt = pot.numb_types()
     fit = 2.0 * (Dn * F0 + F0 * F1 + F1 * F2 + F2) + 2.0 * (F2 * F1 + F1 * F0 + F0 * Dn)
     es = 4.0 if mixed else 8.0
     work = {
@@ -74,21 +74,16 @@ def flops_bytes(pot, n_real, nloc, mixed=False):
         "embed_fwd": ("byte", 4.0 * n_real + (24.0 + es * 4 * L3) * nloc),
         "embed_bwd": ("byte", 4.0 * n_real + (24.0 + es * 4 * L3 + 96.0) * nloc),
         "fitting": ("flop", fit * nloc),
-        # a pass reading dE/dD and T, writing dE/dT, only where the fitting's
-        # fused input-gradient kernel does not apply (axis 16 and F0 240 it
-        # does, in both precisions)
+        # a pass reading dE/dD and T, writing dE/dT
         "dE_dT": ("byte", es * nloc * (Dn + 4 * L3 + 4 * L3)),
         # the edges are scattered inside the embedding backward (fixed point);
-        # this stage folds ghost sums onto owners and assembles per atom the
-        # section sums (96 B per section), the fixed-point force (24 B), the
-        # force (24 B) and the centre partials (96 B)
-        "force": ("byte", (96.0 * nt + 24.0 + 24.0 + 96.0) * nloc),
+        # this stage folds ghost sums onto owners and reads per atom the
+        # centre's own sums (96 B) and the fixed-point force (24 B), and writes
+        # the force (24 B)
+        "force": ("byte", (96.0 + 24.0 + 24.0) * nloc),
         "nlist": ("byte", 4.0 * nloc * pot.nnei + 24.0 * nloc),
     }
-    if nt > 1:
-        # reads the section sums, writes T (the first fitting GEMM forms D from T)
-        work["descriptor"] = ("byte", es * nloc * (nt * 4 * L3 + 4 * L3))
-    if M2 == 16 and F0 == 240:
+    if pot.fitting_form() != FIT_PLAIN:
         del work["dE_dT"]
     return work
 
@@ -228,7 +223,9 @@ def run_config(dp, hip, config, steps, warmup, atomic=False):
         if k in work and t > 0:
             priced(entry, *work[k], t, peak_mfma)
         elif k == "dE_dT" and k not in work:
-            entry["note"] = "fused into the fitting stage's input-gradient kernel"
+            entry["note"] = "formed inside the fitting stage"
+        elif k == "descriptor":
+            entry["note"] = "no pass: the embedding forward writes T"
         stages[k] = entry
     return dict(n=n, ms=ms, ms_sync=ms_sync, ms_host=ms_host, ms_atomic=ms_atomic,
                 stage_ms=stage_ms, stages=stages,
@@ -492,7 +489,7 @@ def main():
     us_atom = main_r["ms"] * 1e3 / n
     ns_day = DT_FS[args.config] * 1e-6 * 86400.0 / (main_r["ms"] * 1e-3)
     # dominant stage (the fitting's six launches are timed as one)
-    kernel_stages = [k for k in ("fitting", "embed_bwd", "embed_fwd", "descriptor", "dE_dT", "nlist")
+    kernel_stages = [k for k in ("fitting", "embed_bwd", "embed_fwd", "dE_dT", "nlist")
                      if k in main_r["work"]]
     dom = max(kernel_stages, key=lambda k: main_r["stage_ms"].get(k, 0.0))
     kind, amount = main_r["work"][dom]
