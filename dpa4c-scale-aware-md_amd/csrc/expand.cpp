@@ -3,11 +3,15 @@
 // the kernels read.
 #include "expand.h"
 
+#include <pthread.h>
+
 #include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <condition_variable>
 #include <exception>
-#include <thread>
+#include <mutex>
+#include <type_traits>
 
 #include "model.h"
 
@@ -52,23 +56,26 @@ void columns(const ld* x, int in, const double* W, int out, ld* z) {
   for (int c = 0; c < C; ++c) z[c] = a[c];
 }
 
-// One net at s, in extended precision (x, y: scratch of at least L3 values).
-void net_ld(const ModelHost& m, const double* P, ld s, std::vector<ld>& x, std::vector<ld>& y) {
+// One net at s, in extended precision: features [L3].
+constexpr int kWidest = 128;
+void net_ld(const ModelHost& m, const double* P, ld s, ld* features) {
   const int L[4] = {1, m.emb[0], m.emb[1], m.emb[2]};
+  ld buf[2][kWidest], *x = buf[0], *y = buf[1];
   x[0] = s;
   for (int k = 0; k < 3; ++k) {
     const int in = L[k], out = L[k + 1];
     const double* W = P;
     const double* b = P + (long)in * out;
     P = b + out;
-    std::copy_n(b, out, y.begin());
+    std::copy_n(b, out, y);
     int f = 0;
-    for (; f + 4 <= out; f += 4) columns<4>(x.data(), in, W + f, out, y.data() + f);
-    for (; f < out; ++f) columns<1>(x.data(), in, W + f, out, y.data() + f);
+    for (; f + 4 <= out; f += 4) columns<4>(x, in, W + f, out, y + f);
+    for (; f < out; ++f) columns<1>(x, in, W + f, out, y + f);
     for (f = 0; f < out; ++f)
       y[f] = tanh_ld(y[f]) + (out == in && k > 0 ? x[f] : out == 2 * in && k > 0 ? x[f % in] : 0.0L);
     std::swap(x, y);
   }
+  std::copy_n(x, L[3], features);
 }
 
 // c_0 .. c_{n-1} over T_k (stride F values) -> the same polynomial over
@@ -83,31 +90,94 @@ void to_products(ld* c, int n, int S, int F) {
       }
 }
 
-// f(0) .. f(n - 1) over the host's cores (up to 8). What an f throws ends the
-// others' work too and is thrown again once every thread has.
-template <class Fn>
-void parallel(int n, Fn&& f) {
-  std::atomic<int> next{0};
-  std::atomic<bool> failed{false};
-  std::exception_ptr error;  // written by the thread that sets failed
-  auto work = [&]() {
-    try {
-      for (int k = next++; k < n && !failed; k = next++) f(k);
-    } catch (...) {
-      if (!failed.exchange(true)) error = std::current_exception();
-    }
-  };
-  std::vector<std::thread> pool;
-  try {
-    pool.reserve(7);
-    for (int q = 1; q < std::min(n, 8); ++q) pool.emplace_back(work);
-  } catch (const std::exception&) {
-    // fewer threads than asked for: the rest of the work stays here
+// The host threads of one build (up to 8 with the caller's), started once: a
+// start costs as much as a phase of a small model. Their stacks are small, so
+// that the C library keeps them for the next build: stacks of the default 8 MB
+// are mostly unmapped, and the device allocations of the handle's first
+// evaluation then land at addresses the card has no page tables for yet (1.3
+// against 0.5 ms for 864 Cu atoms where a handle replaces another).
+class Team {
+ public:
+  Team() {
+    pthread_attr_t attr;
+    if (pthread_attr_init(&attr) != 0) return;
+    (void)pthread_attr_setstacksize(&attr, 256 * 1024);
+    // (if fewer threads than asked for: their work stays with the caller)
+    while (size_ < kThreads && pthread_create(&pool_[size_], &attr, serve, this) == 0) ++size_;
+    (void)pthread_attr_destroy(&attr);
   }
-  work();
-  for (auto& t : pool) t.join();
-  if (error) std::rethrow_exception(error);
-}
+  ~Team() {
+    {
+      std::lock_guard<std::mutex> lock(m_);
+      stop_ = true;
+    }
+    wake_.notify_all();
+    for (size_t q = 0; q < size_; ++q) pthread_join(pool_[q], nullptr);
+  }
+  Team(const Team&) = delete;
+  Team& operator=(const Team&) = delete;
+
+  // f(0) .. f(n - 1), in any order. What an f throws ends the others' work too
+  // and is thrown again once every thread has stopped.
+  template <class Fn>
+  void run(int n, Fn&& f) {
+    {
+      std::lock_guard<std::mutex> lock(m_);
+      call_ = [](void* g, int k) { (*static_cast<std::remove_reference_t<Fn>*>(g))(k); };
+      f_ = &f;
+      n_ = n;
+      next_ = 0;
+      failed_ = false;
+      error_ = nullptr;
+      busy_ = size_;
+      ++round_;
+    }
+    wake_.notify_all();
+    work();
+    std::unique_lock<std::mutex> lock(m_);
+    done_.wait(lock, [this]() { return busy_ == 0; });
+    if (error_) std::rethrow_exception(error_);
+  }
+
+ private:
+  void work() {
+    try {
+      for (int k = next_++; k < n_ && !failed_; k = next_++) call_(f_, k);
+    } catch (...) {
+      if (!failed_.exchange(true)) error_ = std::current_exception();
+    }
+  }
+  static void* serve(void* self) {
+    Team& t = *static_cast<Team*>(self);
+    long seen = 0;
+    std::unique_lock<std::mutex> lock(t.m_);
+    for (;;) {
+      t.wake_.wait(lock, [&]() { return t.stop_ || t.round_ != seen; });
+      if (t.stop_) return nullptr;
+      seen = t.round_;
+      lock.unlock();
+      t.work();
+      lock.lock();
+      if (--t.busy_ == 0) t.done_.notify_one();
+    }
+  }
+
+  static constexpr size_t kThreads = 7;
+  std::mutex m_;
+  std::condition_variable wake_, done_;
+  pthread_t pool_[kThreads];
+  size_t size_ = 0;
+  // the phase: set by run() under the lock, before the threads are woken
+  void (*call_)(void*, int) = nullptr;
+  void* f_ = nullptr;
+  int n_ = 0;
+  std::atomic<int> next_{0};
+  std::atomic<bool> failed_{false};
+  std::exception_ptr error_;  // written by the thread that sets failed_
+  size_t busy_ = 0;           // threads that have not finished the phase
+  long round_ = 0;
+  bool stop_ = false;
+};
 
 // Chebyshev coefficients [n][L3] of the nets of `pairs` from n nodes (even),
 // and per pair the number of terms (a multiple of 16, 0 if none will do) past
@@ -117,7 +187,8 @@ void parallel(int n, Fn&& f) {
 // last 16 coefficients come first: where they alone are larger than that (excess,
 // their sum in units of it, above 1), no number of terms will do, and the others
 // are not formed.
-void coefficients(const ModelHost& m, const std::vector<int>& pairs, int n,
+constexpr int kMostNodes = 304;
+void coefficients(Team& team, const ModelHost& m, const std::vector<int>& pairs, int n,
                   std::vector<std::vector<ld>>& coef, std::vector<int>& terms,
                   std::vector<ld>& excess) {
   constexpr int C = 4;  // features formed together (L3 is a multiple)
@@ -126,21 +197,19 @@ void coefficients(const ModelHost& m, const std::vector<int>& pairs, int n,
   std::vector<ld> cosine(4 * n);  // cos(i pi / 2n): exact angles for cos(k (2j + 1) pi / 2n)
   for (int i = 0; i < 4 * n; ++i) cosine[i] = std::cos((ld)i * pi / (2 * n));
   std::vector<ld> val((size_t)np * n * F);  // [pair][node][feature]
-  parallel(np * n, [&](int k) {
+  for (int p : pairs) coef[p].assign((size_t)n * F, 0.0L);
+  team.run(np * n, [&](int k) {
     const int p = pairs[k / n], j = k % n;
     const ld z = (cosine[2 * j + 1] + (ld)kExpandB) / (ld)kExpandA;
     const ld s = (z / (2 - z) / (ld)kExpandRmin - (ld)m.davg[(size_t)p * 4]) / (ld)m.dstd[(size_t)p * 4];
-    std::vector<ld> x(F), y(F);
-    net_ld(m, m.emb_params.data() + (size_t)p * m.emb_block, s, x, y);
-    std::copy_n(x.begin(), F, val.begin() + (size_t)k * F);
+    net_ld(m, m.emb_params.data() + (size_t)p * m.emb_block, s, val.data() + (size_t)k * F);
   });
-  for (int p : pairs) coef[p].assign((size_t)n * F, 0.0L);
   // coefficients k0 .. k1 - 1 of features C q .. C q + C - 1 of pair pairs[i]
   auto transform = [&](int i, int q, int k0, int k1) {
     const ld* v = val.data() + (size_t)i * n * F + C * q;
     ld* c = coef[pairs[i]].data() + C * q;
     // node n - 1 - j lies opposite node j: T_k there is (-1)^k T_k here
-    std::vector<ld> fold((size_t)n * C);
+    ld fold[kMostNodes * C];
     for (int j = 0; j < n / 2; ++j)
       for (int f = 0; f < C; ++f) {
         const ld a = v[(size_t)j * F + f], b = v[(size_t)(n - 1 - j) * F + f];
@@ -148,7 +217,7 @@ void coefficients(const ModelHost& m, const std::vector<int>& pairs, int n,
         fold[(n / 2 + j) * C + f] = a - b;
       }
     for (int k = k0; k < k1; ++k) {
-      const ld* w = fold.data() + (k % 2 ? n / 2 * C : 0);
+      const ld* w = fold + (k % 2 ? n / 2 * C : 0);
       ld sum[C] = {};
       int at = k;  // k (2j + 1) mod 4n
       for (int j = 0; j < n / 2; ++j) {
@@ -170,9 +239,9 @@ void coefficients(const ModelHost& m, const std::vector<int>& pairs, int n,
     }
     return sum;
   };
-  parallel(np * NF, [&](int q) { transform(q / NF, q % NF, n - 16, n); });
+  team.run(np * NF, [&](int q) { transform(q / NF, q % NF, n - 16, n); });
   std::vector<ld> limit(np, 0.0L), last(np);
-  parallel(np, [&](int i) {
+  team.run(np, [&](int i) {
     for (size_t k = 0; k < (size_t)n * F; ++k)
       limit[i] = std::max(limit[i], std::fabs(val[(size_t)i * n * F + k]));
     limit[i] *= 0x1p-55L;
@@ -184,7 +253,7 @@ void coefficients(const ModelHost& m, const std::vector<int>& pairs, int n,
     if (last[i] <= limit[i]) good.push_back(i);
     else excess[pairs[i]] = limit[i] > 0 ? last[i] / limit[i] : last[i];
   }
-  parallel((int)good.size() * NF, [&](int q) { transform(good[q / NF], q % NF, 0, n - 16); });
+  team.run((int)good.size() * NF, [&](int q) { transform(good[q / NF], q % NF, 0, n - 16); });
   for (int i : good) {
     ld sum = last[i];
     for (int k = n - 16; k >= 16 && sum <= limit[i]; k -= 16) {
@@ -204,11 +273,12 @@ bool build_expansion(const ModelHost& m, ExpandHost& e) {
       if (!std::isfinite(x)) return false;
   std::vector<std::vector<ld>> coef(np);
   std::vector<int> terms(np, 0);
+  Team team;
   std::vector<ld> excess(np, 0.0L);
   std::vector<int> todo(np);
   for (int p = 0; p < np; ++p) todo[p] = p;
   auto expand = [&](const std::vector<int>& pairs, int n) {
-    coefficients(m, pairs, n, coef, terms, excess);
+    coefficients(team, m, pairs, n, coef, terms, excess);
     todo.clear();
     for (int p = 0; p < np; ++p)
       if (terms[p] == 0) todo.push_back(p);
@@ -219,10 +289,10 @@ bool build_expansion(const ModelHost& m, ExpandHost& e) {
     // a model that has none costs little more than the first attempt
     const int worst = *std::max_element(todo.begin(), todo.end(),
                                         [&](int p, int q) { return excess[p] < excess[q]; });
-    expand({worst}, 304);
+    expand({worst}, kMostNodes);
     if (terms[worst] == 0) return false;
   }
-  for (const int n : {176, 304})
+  for (const int n : {176, kMostNodes})
     if (!todo.empty()) expand(std::vector<int>(todo), n);
   if (!todo.empty()) return false;
   const int most = *std::max_element(terms.begin(), terms.end());
@@ -232,13 +302,14 @@ bool build_expansion(const ModelHost& m, ExpandHost& e) {
   e.fwd.assign((size_t)np * fs, 0.0);
   e.bwd.assign((size_t)np * bs, 0.0);
   e.blocks.assign(np, 0);
-  parallel(np, [&](int p) {
+  std::vector<ld> prod((size_t)np * N * F, 0.0L);
+  team.run(np, [&](int p) {
     e.blocks[p] = terms[p] / 16;
-    std::vector<ld> c((size_t)N * F, 0.0L);
-    std::copy_n(coef[p].begin(), (size_t)terms[p] * F, c.begin());
-    to_products(c.data(), N, 64, F);
-    for (int h = 0; h < N; h += 64) to_products(c.data() + (size_t)h * F, 64, 16, F);
-    for (int h = 0; h < N; h += 16) to_products(c.data() + (size_t)h * F, 16, 4, F);
+    ld* c = prod.data() + (size_t)p * N * F;
+    std::copy_n(coef[p].begin(), (size_t)terms[p] * F, c);
+    to_products(c, N, 64, F);
+    for (int h = 0; h < N; h += 64) to_products(c + (size_t)h * F, 64, 16, F);
+    for (int h = 0; h < N; h += 16) to_products(c + (size_t)h * F, 16, 4, F);
     // (a product expansion of a polynomial of degree < 16 blocks has no terms
     // beyond those blocks: each conversion only moves weight downwards)
     for (int k = 0; k < N; ++k)
