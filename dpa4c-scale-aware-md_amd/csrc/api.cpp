@@ -26,6 +26,7 @@
 #include <cmath>
 #include <cstring>
 #include <fstream>
+#include <future>
 #include <iterator>
 #include <string>
 #include <type_traits>
@@ -90,8 +91,9 @@ struct dp_model {
   void* d_c4 = nullptr;  // every DPA4C parameter array, packed
   EmbLayout el{};
   std::string err;
-  // device parameters; the nets (d_emb, d_fit) are double in fp64 mode and
-  // float in mixed mode, env statistics and the padded-slot constant are fp64
+  // device parameters; the nets (d_emb, only of models without an expansion, and
+  // d_fit) are double in fp64 mode and float in mixed mode, env statistics and the
+  // padded-slot constant are fp64
   void* d_emb = nullptr;
   double* d_envp = nullptr;
   double* d_tpad = nullptr;
@@ -1460,6 +1462,14 @@ int dp_create(const char* path, int gpu_rank, const void* file_content, size_t c
     const ModelHost& m = M->host;
     const bool mixed = precision == DP_PREC_MIXED;
     M->el = make_emb_layout(m.emb[0], m.emb[1], m.emb[2], mixed);
+    // the expansion is built beside the packing of the other parameters (with it
+    // after them, and the nets packed for both evaluations, dp_create took 20 / 34 ms
+    // for HEA in fp64 / mixed, 6.3 for water and 2.3 for Cu; now 12 / 23, 4.6, 1.4)
+    auto expansion = std::async(std::launch::async | std::launch::deferred, [&m]() {
+      ExpandHost ex;
+      if (!build_expansion(m, ex)) ex.H = 0;
+      return ex;
+    });
     std::vector<double> emb, envp, tpad;
     pack_embedding(m, M->el, emb, envp, tpad);
     auto upload = [&](auto*& dst, const auto& src) {
@@ -1472,20 +1482,7 @@ int dp_create(const char* path, int gpu_rank, const void* file_content, size_t c
     };
     upload(M->d_envp, envp);
     upload(M->d_tpad, tpad);
-    ExpandHost ex;
-    if (build_expansion(m, ex)) {
-      M->exp_h = ex.H;
-      M->exp_blocks = ex.blocks;
-      upload(M->d_exp_f, ex.fwd);
-      upload(M->d_exp_b, ex.bwd);
-      upload(M->d_exp_pad, ex.phi_pad);
-      upload(M->d_nets, m.emb_params);
-    }
     if (mixed) {
-      // the nets are evaluated in fp32: round the parameters once here
-      std::vector<float> emb32(emb.begin(), emb.end());
-      pack_embedding_bf16(m, M->el, emb32);
-      upload(M->d_emb, emb32);
       // fitting GEMM operands pre-split for the bf16 matrix cores: W0, W1,
       // W2 forward, W1 / W2 transposed, and W0 transposed tile-major for the
       // fused dE/dD -> dE/dT kernel (when it applies; otherwise dE/dD is
@@ -1505,8 +1502,6 @@ int dp_create(const char* path, int gpu_rank, const void* file_content, size_t c
                            m.fit[k], tr == 1, frag, k == 0 && tr == 1);
           }
       upload(M->d_fitf, frag);
-    } else {
-      upload(M->d_emb, emb);
     }
     M->fo = fit_offsets(m);
     {
@@ -1541,6 +1536,22 @@ int dp_create(const char* path, int gpu_rank, const void* file_content, size_t c
         upload(M->d_fit, padded(0.0));
         upload(M->d_fit_t, transposed(0.0));
       }
+    }
+    const ExpandHost ex = expansion.get();
+    if (ex.H > 0) {
+      M->exp_h = ex.H;
+      M->exp_blocks = ex.blocks;
+      upload(M->d_exp_f, ex.fwd);
+      upload(M->d_exp_b, ex.bwd);
+      upload(M->d_exp_pad, ex.phi_pad);
+      upload(M->d_nets, m.emb_params);
+    } else if (mixed) {
+      // the nets are evaluated slot by slot in fp32: round the parameters once here
+      std::vector<float> emb32(emb.begin(), emb.end());
+      pack_embedding_bf16(m, M->el, emb32);
+      upload(M->d_emb, emb32);
+    } else {
+      upload(M->d_emb, emb);
     }
     M->bytes_peak = M->bytes_now;
     if (const char* g = std::getenv("DPAMD_GRAPH")) M->graph_on = std::atoi(g) != 0;
